@@ -186,7 +186,11 @@ PMI_API int pmi_tile_w4a16(const uint8_t* w_kernel, uint8_t* w_tiled, int64_t N,
  * its first use; every call leaves it zero-filled again (it holds split-K
  * counters, partial tiles and the act_order gather of X). A smaller or null
  * workspace is accepted: the GEMM then runs without split-K, and act_order
- * shapes fall back to the GEMV. Calls that may run concurrently (other
+ * shapes fall back to the GEMV. With pmi_matmul_best_workspace_bytes() bytes,
+ * row counts past 11 that would stream the weights once per four (GEMV) or 64
+ * rows (bf16, group sizes 32 and 64, K % 256 != 0, callers without w_tiled) run
+ * on the big-tile GEMM where that wins (N % 4 == 0, K % 128 == 0, y 8-byte
+ * aligned). Calls that may run concurrently (other
  * streams) must not share a workspace.
  * Requires K % group_size == 0, group_size % 32 == 0, K % 32 == 0.
  * Replaces: matmul_w4a16(x, packed_weight, scales, zeros, group_size)
@@ -200,7 +204,8 @@ PMI_API int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const
 /* pmi_matmul_w4a16 without a workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). Same arguments, kernels and results as
- * pmi_matmul_w4a16 given a workspace of pmi_matmul_workspace_bytes() bytes.
+ * pmi_matmul_w4a16 given the scratch as its workspace (none where
+ * pmi_matmul_workspace_bytes() is 0).
  * The scratch is a fixed 16 MiB array the library holds on each GPU it runs
  * on until the process ends (found with hipGetSymbolAddress on the first call
  * on a device, which also clears its counter block: make that first call
@@ -332,6 +337,12 @@ PMI_API int pmi_tiled_rmsnorm_supported(int64_t M, int64_t N, int64_t K, int64_t
  * Triton kernel allocates nothing besides Y (pare/kernels/matmul_int4.py:230). */
 PMI_API size_t pmi_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size,
                                   int has_perm);
+
+/* At least pmi_matmul_workspace_bytes(): also what the big-tile GEMM uses for
+ * calls that run on another kernel without it (bf16 row sums, group-major
+ * copies, split-K partial tiles). Host-only. No reference counterpart. */
+PMI_API size_t pmi_matmul_best_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size,
+                                               int has_perm);
 
 /* Full dequantised weight W_hat[N,K] in the original column order, cast to
  * out_dtype (PMI_F16 / PMI_BF16 with round-to-nearest-even, or PMI_F32).

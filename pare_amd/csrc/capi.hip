@@ -470,6 +470,114 @@ size_t tgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size
   return xg + split ? pmi::kWsCounterBytes + xg + split : 0;
 }
 
+// ---- where the big-tile GEMM runs beside choice 6 -----------------------------
+// (its choice for fp16 with the tiled copy and group sizes that are multiples
+// of 128). In its place the calls below ran the GEMV four activation rows at a
+// time, the tiled GEMM 64 rows at a time, or the register-streamed GEMM.
+
+// GEMV calls of many rows: no other kernel reads the shape's group size or
+// column count, or x is bf16. The GEMV streams the weights once per four rows
+// (4096 x 4096: 5.3 us each), the big-tile GEMM takes 15-25 us for any few rows
+// (gs 64, M = 16 / 32: 22 / 43 against 21 / 22 us; 14336 x 4096, M = 16: 61
+// against 30).
+bool bgemm_over_gemv(int64_t M, int64_t N, int64_t K) {
+  return M > 24 || (M >= 12 && N * K >= (1ll << 25));
+}
+
+// Group sizes 32 and 64 on the tiled copy, past 64 rows (tiled GEMM / big-tile,
+// us, gs 64): 4096 x 4096 at M = 128 / 192 / 512 21.3 / 29.1 / 75 against 23.4 /
+// 24.6 / 35.5; 1024 x 4096 at M = 512 / 768 21.4 / 33.0 against 24.3 / 24.5; 4096 x
+// 14336 at M = 65 / 512 50 / 227 against 30 / 81; 14336 x 4096 at M = 256 54.8
+// against 58.5 (a third block of 112 rows nearly empty), at M = 384 82 against 61.
+bool bgemm_over_tgemm(int64_t M, int64_t N, int64_t K, const pmi::BgemmConfig& b) {
+  if (M <= 64 || M * N * K < 3000000000ll) return false;
+  if (K > 8192) return true;
+  if (M < 192) return false;
+  return (int64_t)b.n_bands * b.grid_m * 2 <= pmi::device_cu_count() || M > 384 ||
+         (int64_t)b.grid_m * 16 * b.mt * 5 <= 6 * M;
+}
+
+// 128-column groups without the tiled copy, against the register-streamed GEMM
+// (us). With the group-major copies: 14336 x 4096 at M = 384 / 512 60.5 / 90 against
+// 64.5 / 66.9, so from tiles for three quarters of the CUs. Without them (which
+// slows that kernel, and costs the big-tile GEMM a 3-5 us launch that makes
+// them): 4096 x 4096 at M = 512 / 768 28.7 / 53 against 33 / 45, 14336 x 4096 at
+// M = 256 / 384 52 / 78 against 47 / 64.5, 4096 x 14336 at M = 256 / 384 47 / 74.5
+// against 44 / 58.8.
+bool bgemm_over_gemm64(int64_t M, int64_t N, int64_t K, bool has_gm, const pmi::BgemmConfig& b) {
+  if (M <= 64) return false;
+  if (has_gm) return (int64_t)b.n_bands * b.grid_m * 4 >= 3 * pmi::device_cu_count();
+  return M * N * K > (1ll << 34);
+}
+
+// Whether a call whose kernel is otherwise `choice` runs on the big-tile GEMM;
+// tiled and gm: the copies it was given.
+bool use_bgemm(int choice, bool bf16, bool tiled, bool gm, int64_t M, int64_t N, int64_t K, int64_t gs) {
+  if (choice == 6 && !bf16) return true;
+  if (M < 12 || (!tiled && gs != 32 && gs != 64 && gs != 128)) return false;
+  const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, gs, bf16);
+  if (!b.ok) return false;
+  if (bf16 || choice == 1) return bgemm_over_gemv(M, N, K);
+  if (choice == 5) return tiled && gs < 128 && bgemm_over_tgemm(M, N, K, b);
+  return (choice == 2 || choice == 4) && gs == 128 && !tiled && bgemm_over_gemm64(M, N, K, gm, b);
+}
+
+// Group-major copies made in the workspace for callers without them.
+size_t ws_sz_bytes(int64_t N, int64_t K, int64_t gs) {
+  return pmi::ws_align((size_t)N * (K / gs) * 4) + pmi::ws_align((size_t)N * (K / gs));
+}
+
+// Workspace that lets the big-tile GEMM take the calls above and split K (with
+// less they run as they would without it, or unsplit).
+size_t bgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t gs, bool has_perm) {
+  if (M < 12) return 0;
+  size_t need = 0;
+  for (int bf16 = 0; bf16 < 2; ++bf16) {
+    const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, gs, bf16);
+    if (!b.ok) return 0;
+    for (int t = 0; t < 2; ++t) {
+      const int flags = (t ? PMI_CHOICE_TILED : 0) | (has_perm ? PMI_CHOICE_PERM : 0);
+      if (!use_bgemm(pmi_matmul_kernel_choice(M, N, K, gs, flags), bf16, t, t, M, N, K, gs)) continue;
+      const size_t n = b.ws_sums + b.ws_split + (t ? 0 : ws_sz_bytes(N, K, gs));
+      need = n > need ? n : need;
+    }
+  }
+  return need ? pmi::kWsCounterBytes + (has_perm ? pmi::ws_perm_bytes(M, K) : 0) + need : 0;
+}
+
+// Runs the big-tile GEMM: X[:, perm] gathered first with act_order, the
+// group-major copies made in the workspace where gm is false. *ran = false (and
+// nothing launched) when the workspace is too small for what it cannot do
+// without.
+hipError_t run_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w, const float* scales,
+                     const void* zeros, int zero_u8, const float* scales_gm, const uint8_t* zeros_gm,
+                     const int32_t* perm, void* y, int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16,
+                     void* workspace, size_t ws_bytes, hipStream_t s, bool* ran) {
+  const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, gs, bf16);
+  const bool gm = scales_gm && zeros_gm;
+  size_t off = pmi::kWsCounterBytes;
+  const size_t perm_off = off;
+  if (perm) off += pmi::ws_perm_bytes(M, K);
+  const size_t sz_off = off;
+  if (!gm) off += ws_sz_bytes(N, K, gs);
+  *ran = off + b.ws_sums == pmi::kWsCounterBytes || (workspace && ws_bytes >= off + b.ws_sums);
+  if (!*ran) return hipSuccess;
+  uint8_t* ws = (uint8_t*)workspace;
+  if (perm) {
+    if (hipError_t e = pmi::launch_gather_cols(x, perm, ws + perm_off, M, K, s); e != hipSuccess) return e;
+    x = ws + perm_off;
+  }
+  if (!gm) {
+    float* s_out = (float*)(ws + sz_off);
+    uint8_t* z_out = ws + sz_off + pmi::ws_align((size_t)N * (K / gs) * 4);
+    if (hipError_t e = pmi::launch_sz_group_major(scales, zeros, zero_u8, 0, s_out, z_out, nullptr, N, K / gs, s);
+        e != hipSuccess)
+      return e;
+    scales_gm = s_out, zeros_gm = z_out;
+  }
+  return pmi::launch_bgemm(x, w_tiled, w, scales_gm, zeros_gm, y, M, N, K, gs, bf16, workspace, ws_bytes, off, s);
+}
+
 size_t other_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size, int has_perm) {
   const int choice = pmi_matmul_kernel_choice(M, N, K, group_size, 0);
   if (choice == 2 && pmi::gemm_supported(K, group_size))
@@ -514,6 +622,14 @@ size_t pmi_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group
   return need;
 }
 
+size_t pmi_matmul_best_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size,
+                                       int has_perm) {
+  const size_t base = pmi_matmul_workspace_bytes(M, N, K, group_size, has_perm);
+  if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || K % group_size != 0) return base;
+  const size_t big = bgemm_workspace_bytes(M, N, K, group_size, has_perm != 0);
+  return big > base ? big : base;
+}
+
 int pmi_sz_group_major(const float* scales, const void* zeros, int zero_dtype, float* scales_gm,
                        uint8_t* zeros_gm, int32_t* bad_count, int64_t N, int64_t G,
                        void* stream) {
@@ -523,7 +639,7 @@ int pmi_sz_group_major(const float* scales, const void* zeros, int zero_dtype, f
   if (N * G >= (1ll << 31)) return fail(PMI_ERR_UNSUPPORTED, "%s: N*G too large", fn);
   if (N == 0) return ok();
   if (!scales || !zeros || !scales_gm || !zeros_gm) return fail(PMI_ERR_INVALID, "%s: null buffer", fn);
-  return from_hip(pmi::launch_sz_group_major(scales, zeros, zero_dtype == PMI_U8, scales_gm,
+  return from_hip(pmi::launch_sz_group_major(scales, zeros, zero_dtype == PMI_U8, 1, scales_gm,
                                              zeros_gm, bad_count, N, G, (hipStream_t)stream),
                   fn);
 }
@@ -585,6 +701,14 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
       return from_hip(pmi::launch_tgemm(x, nullptr, nullptr, w_tiled, scales_gm, zeros_gm, y, M, N,
                                         K, group_size, nullptr, 0, 0, s, true),
                       fn);
+    // many rows: the big-tile GEMM, from the tiled copy where there is one
+    const bool gm = scales_gm && zeros_gm;
+    if (!forced && aligned(y, 8) && use_bgemm(1, true, gm && w_tiled, gm, M, N, K, group_size)) {
+      bool ran = false;
+      const hipError_t e = run_bgemm(x, gm ? w_tiled : nullptr, w, scales, zeros, zu8, scales_gm, zeros_gm, perm, y,
+                                     M, N, K, group_size, true, workspace, workspace_bytes, s, &ran);
+      if (ran) return from_hip(e, fn);
+    }
     const uint16_t* xp = (const uint16_t*)x;
     if (perm) {
       if (workspace_bytes < pmi::kWsCounterBytes + pmi::ws_perm_bytes(M, K))
@@ -621,18 +745,20 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
         !pmi::bgemm_config(M, N, K, group_size).ok)
       return fail(PMI_ERR_UNSUPPORTED, "%s: the big-tile GEMM needs w_tiled, scales_gm and zeros_gm, "
                   "N %% 4 == 0, K %% 512 == 0, K >= 1536, group_size %% 128 == 0 and M * K < 2^30", fn);
-    // act_order: X[:, perm] gathered into the workspace first
-    const void* xs = x;
-    if (perm) {
-      if (workspace_bytes < pmi::kWsCounterBytes + pmi::ws_perm_bytes(M, K))
-        return fail(PMI_ERR_UNSUPPORTED, "%s: the big-tile GEMM with perm needs a workspace of "
-                    "pmi_matmul_workspace_bytes() bytes", fn);
-      void* xg = (uint8_t*)workspace + pmi::kWsCounterBytes;
-      hipError_t e = pmi::launch_gather_cols(x, perm, xg, M, K, s);
-      if (e != hipSuccess) return from_hip(e, fn);
-      xs = xg;
-    }
-    return from_hip(pmi::launch_bgemm(xs, w_tiled, scales_gm, zeros_gm, y, M, N, K, group_size, s), fn);
+    bool ran = false;
+    const hipError_t e = run_bgemm(x, w_tiled, w, scales, zeros, zu8, scales_gm, zeros_gm, perm, y, M, N, K,
+                                   group_size, false, workspace, workspace_bytes, s, &ran);
+    if (!ran)
+      return fail(PMI_ERR_UNSUPPORTED, "%s: the big-tile GEMM with perm needs a workspace of "
+                  "pmi_matmul_workspace_bytes() bytes", fn);
+    return from_hip(e, fn);
+  }
+  const bool gm = scales_gm && zeros_gm;
+  if (!forced && aligned(y, 8) && use_bgemm(choice, false, has_tiled, gm, M, N, K, group_size)) {
+    bool ran = false;
+    const hipError_t e = run_bgemm(x, has_tiled ? w_tiled : nullptr, w, scales, zeros, zu8, scales_gm, zeros_gm,
+                                   perm, y, M, N, K, group_size, false, workspace, workspace_bytes, s, &ran);
+    if (ran) return from_hip(e, fn);
   }
   if (choice == 5) {
     if (!has_tiled || !pmi::tgemm_supported(M, N, K, group_size))
@@ -806,6 +932,8 @@ int pmi_matmul_w4a16_noalloc(const void* x, int x_dtype, const uint8_t* w, const
                 "K=%lld%s), more than the library's fixed %zu; call pmi_matmul_w4a16 with a "
                 "workspace of pmi_matmul_workspace_bytes() bytes", fn, need, (long long)M,
                 (long long)N, (long long)K, perm ? ", act_order" : "", kScratchBytes);
+  // (calls that need no scratch are given none, so that they stay free to
+  // overlap: the big-tile GEMM's optional workspace is not taken from it)
   void* ws = nullptr;
   if (need) {
     if (int rc = scratch_ptr(&ws, (hipStream_t)stream, fn)) return rc;

@@ -151,8 +151,9 @@ hipError_t launch_gemm(const void* x, const uint8_t* w, const float* scales, con
                        void* workspace, size_t ws_bytes, hipStream_t stream);
 
 // [N, G] scales and zero points -> group-major fp32 [G, N] and u8 [G, N]
-// (zeros must hold integers in [0, 15]; others are counted into *bad).
-hipError_t launch_sz_group_major(const float* scales, const void* zeros, int zero_u8,
+// (strict: zeros must hold integers in [0, 15], others are counted into *bad
+// and become 0; otherwise they are taken as the matmul kernels take them).
+hipError_t launch_sz_group_major(const float* scales, const void* zeros, int zero_u8, int strict,
                                  float* scales_gm, uint8_t* zeros_gm, int32_t* bad, int64_t N,
                                  int64_t G, hipStream_t stream);
 
@@ -242,20 +243,28 @@ bool tgemm_supported(int64_t M, int64_t N, int64_t K, int64_t gs);
 constexpr int kTgemmXGLds = 160 * 1024 - 1024;
 bool tgemm_gather_supported(int64_t M, int64_t K);
 TgemmConfig tgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs, bool gather);
-// The big-tile variant of the tiled GEMM (w4a16_bgemm.hip), for many
-// activation rows: 256 weight rows (four panels) x 128 activation rows per
-// workgroup over all of K, B formed as fp16((q - z) * s); no workspace.
+// The big-tile GEMM (w4a16_bgemm.hip), for many activation rows: 256 weight
+// rows (four panels) x 16 mt activation rows per tile; N % 4 == 0, K % 128 == 0,
+// gs 32, 64 or a multiple of 128.
 struct BgemmConfig {
-  bool ok;      // the shape is within the kernel's limits (gs % 128 == 0, K % 128 == 0)
-  int n_bands;  // bands of four 64-row panels
-  int grid_m;   // 128-row activation blocks
-  int chunk;    // (activation block, band) pairs per XCD
-  int grid;     // workgroups (8 chunk)
+  bool ok;         // the shape is within the kernel's limits
+  int mt;          // 16-row activation tiles per workgroup
+  int kg;          // four-wave groups per workgroup that share a tile's K units
+  int n_bands;     // bands of four 64-row panels
+  int grid_m;      // activation blocks
+  int splits;      // workgroups that share a tile's K range
+  int chunk;       // workgroups per XCD
+  int grid;        // workgroups (8 chunk)
+  int sums_ld;     // bf16: floats per row of the row-sum table
+  size_t ws_sums;  // bf16: workspace bytes of the row sums (required)
+  size_t ws_split; // workspace bytes of the partial tiles (without them: unsplit)
 };
-BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs);
-hipError_t launch_bgemm(const void* x, const uint8_t* w_tiled, const float* scales_gm,
+BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16 = false);
+// w_tiled, or (null) the kernel layout w_kernel with gs 32, 64 or 128.
+// workspace: the row sums (bf16) and partial tiles, from ws_offset on.
+hipError_t launch_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w_kernel, const float* scales_gm,
                         const uint8_t* zeros_gm, void* y, int64_t M, int64_t N, int64_t K, int64_t gs,
-                        hipStream_t stream);
+                        bool bf16, void* workspace, size_t ws_bytes, size_t ws_offset, hipStream_t stream);
 // perm: act_order columns, gathered in the kernel (tgemm_gather_supported), or null;
 // perm16 (nullable, with perm): its 16-bit copy, which the gather then reads instead.
 // workspace: counters (zero between calls) at its start and the split-K partial

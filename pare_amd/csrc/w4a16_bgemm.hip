@@ -1,41 +1,57 @@
-// Big-tile GEMM: the tiled-weight INT4 W4A16 GEMM for many activation rows
-// (prefill), gfx950 (v_mfma_f32_16x16x32_f16). A variant of the tiled GEMM
-// (w4a16_tgemm.hip) over the same buffers: tiled weights, group-major scales
-// and zero points.
+// Big-tile GEMM: INT4 W4A16 for many activation rows (prefill), gfx950
+// (v_mfma_f32_16x16x32_f16 / _bf16).
 //
-// Work. A workgroup owns a 256 x 128 output tile (four 64-row weight panels x
-// 128 activation rows) over all of K, with eight compute waves, two per SIMD:
-// wave w takes the 16-row weight tiles 2 (w % 2) and 2 (w % 2) + 1 of panel
-// w / 2 against all 128 activation rows (eight MFMA row tiles). Per 128-column
-// unit a workgroup moves 32 KiB of activations and 16 KiB of codes for 8.4
-// MFLOP; each B operand is formed once and feeds eight MFMAs. Against four
-// panels x two activation halves (every B operand formed by two waves, four
-// MFMAs each) this is 35 % fewer VALU instructions for twice the LDS A-operand
-// reads, and 4-8 % faster (4096 x 4096 at M = 2048: 81 against 85 us). With
-// two waves on a SIMD, one wave's MFMAs can run while the other forms B
-// operands.
+// Work. A group of four waves owns MT 16-row activation tiles x 256 weight
+// rows (a band of four 64-row panels), wave w the 64 rows of panel w against
+// every activation row, over 128-column units of K. Each B operand (8 weights
+// of a lane) is formed once and feeds MT MFMAs; each A operand read from LDS
+// feeds four. Per unit and wave that is 16 MT MFMAs against 16 MT folds (fma
+// x 4 lanes of accumulators), 176 instructions to form the B operands and 4 MT
+// LDS reads. The layout before this one (eight waves of 32 rows x 128) read
+// each A operand for two MFMAs only, which kept the LDS pipe as busy as the
+// matrix cores: 4096 x 28672 x 4096 went from 937 to 745-765 us.
 //
-// Placement. The workgroups are numbered activation block by activation
-// block and dealt to the 8 XCDs in contiguous ranges (the dispatcher deals
-// workgroups round-robin, so workgroup 8 k + x runs on XCD x): the bands that
-// share an activation block share an XCD and read its rows from that XCD's
-// L2. The activation rows are twice the weight bytes of a workgroup, so they
-// are the operand kept local. A placement preference only.
+// Two groups per CU. A wave alternates between forming B operands (VALU) and
+// MFMAs, so a SIMD needs two waves to keep both pipes busy. With KG = 1 a
+// workgroup is one group and two workgroups share a CU (80 KiB of LDS and 256
+// VGPRs each); where the output has no more tiles than the chip has CUs,
+// KG = 2 makes a workgroup of two groups that take alternate units of one tile
+// and add their accumulators through LDS at the end. Where the tiles fill
+// less than half of the CUs, K is also split over workgroups (`splits`), whose
+// fp32 partial tiles a second launch adds in split order.
 //
-// Operands. Each unit's activation rows (128 x 256 bytes), the band's four
-// 4 KiB weight blocks and its scales and zero points go global -> registers
-// -> LDS, double-buffered in LDS: every wave writes its eighth of unit s + 1 to
-// the other slot after computing unit s, then loads the codes of unit s + 2
-// and the activations of unit s + 3 (two register stages for the
-// activations, whose loads otherwise stalled the slot writes; 79 against 81
-// us at 4096 x 4096, M = 2048); one barrier per unit. In a slot, the 16-byte chunk
-// c of activation row r sits at chunk c ^ (r % 16), so the 16 rows an
-// A-operand read touches at one column fall in 16 different bank groups.
+// Staging. Everything goes global -> LDS by buffer_load ... lds, no registers
+// in between: the unit's activation rows (128 columns, 16-byte chunk c of row r
+// at chunk c ^ (r % 16), so the 16 rows of an A read fall in 16 bank groups),
+// double-buffered; the wave's own 4 KiB of codes, single-buffered (they are
+// read into registers at the head of a unit, and the copies of the next unit's
+// follow). One s_barrier per unit. The copies are issued from inline asm: the
+// compiler, which cannot tell the two activation slots apart, would otherwise
+// drain them before every A read. They write LDS only (no register), and each
+// wave waits for its own (vmcnt(0)) before the barrier that publishes them.
 //
-// Numerics: those of the tiled GEMM. B = 8 fp16 (q - z), exact (v_perm_b32
-// under a 0x64 exponent byte, one packed subtract); the products x (q - z)
-// are exact in fp32; per unit y += s * sum x (q - z) in fp32, the reference's
-// w = (q - z) * s with fp32 accumulation (pare/kernels/matmul_int4.py:145-176).
+// Fold. Weight tiles go two at a time: the eight MFMAs of a pair run beside the
+// fold (y += s * sum x (q - z), fp32) of the pair before it, interleaved by
+// sched_group_barrier. Raised wave priority during the MFMAs lets the other
+// wave's B operands fill the gaps (4096 x 28672 x 4096: 773 -> 747 us).
+//
+// Group sizes. KSG = 32-column k-steps per scale group inside a unit: 4 (group
+// sizes that are multiples of 128), 2 (64) and 1 (32), whose scales and zero
+// points are staged in LDS as well (fewer activation rows make room: MT = 7
+// and 6).
+//
+// bf16 (BF). gfx950 has no packed bf16 subtract: B is 128 + q (exact) and a
+// group's sum starts from -(128 + z) * sum x instead of 0; the row sums
+// come from a pass over x ahead of the launch (bgemm_row_sums_kernel).
+//
+// Sources of the codes: the tiled copy (one contiguous 4 KiB block per panel and
+// unit), or (RM) the row-major kernel layout, 64 bytes per row and unit, for
+// callers without the copy.
+//
+// Numerics (fp16): those of the tiled GEMM. B = q - z exact (v_perm_b32 under a
+// 0x64 exponent byte, one packed subtract); the products x (q - z) are exact in
+// fp32; y += s * sum x (q - z) per group in fp32, the reference's w = (q - z) * s
+// with fp32 accumulation (pare/kernels/matmul_int4.py:145-176).
 #include <atomic>
 
 #include "pmi_common.h"
@@ -44,259 +60,614 @@
 namespace pmi {
 namespace {
 
-constexpr int kBWaves = 8;  // compute waves: 4 panels x 2 activation halves
-constexpr int kBMT = 8;     // 16-row activation tiles per wave (all 128 rows)
-// one LDS slot: activations, the four panels' weight blocks, scales, zero points
-constexpr int kBX = 128 * 256;          // 32 KiB: 128 rows x 256 bytes
-constexpr int kBWo = kBX;               // weights: 4 panels x 4 KiB
-constexpr int kBSo = kBWo + 4 * 4096;   // scales: 256 rows x 4 bytes
-constexpr int kBZo = kBSo + 1024;       // zero points: 256 rows x 1 byte
-constexpr int kBSlot = kBZo + 256;
-static_assert(2 * kBSlot <= 160 * 1024, "two slots fit LDS");
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 struct BgemmArgs {
-  const f16* x;
-  const uint8_t* wt;    // tiled weights
-  const float* s_gm;    // fp32 [G, N]
-  const uint8_t* z_gm;  // u8 [G, N]
-  f16* y;
+  const uint16_t* x;     // fp16 or bf16 [M, K]
+  const uint8_t* w;      // tiled weights, or kernel layout [N, K/2] (RM)
+  const float* s_gm;     // fp32 [G, N]
+  const uint8_t* z_gm;   // u8 [G, N]
+  const float* sums;     // BF: row sums of x per scale group of a unit, [.., sums_ld]
+  uint16_t* y;           // [M, N]
+  float* part;           // splits > 1: partial tiles
   int M, N, K, gs;
-  int n_panels;  // 64-row panels of the tiled weights
-  int n_bands;   // bands of four panels
-  int grid_m;    // 128-row activation blocks
-  int chunk;     // (activation block, band) pairs per XCD
+  int n_panels, n_bands, grid_m, splits;
+  int chunk;             // workgroups per XCD
+  int sums_ld;
 };
 
-// s_waitcnt lgkmcnt(0), the other counters left alone (gfx9 encoding)
-PMI_DEV void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xF | 0x70 | (3 << 14)); }
+template <int MT, int KSG, bool BF>
+struct Shape {
+  static constexpr int kRows = 16 * MT;
+  static constexpr int kX = kRows * 256;                  // one activation slot
+  static constexpr int kGU = 4 / KSG;                     // scale groups per unit
+  static constexpr bool kSzLds = KSG < 4 || BF;           // scales and zero points in LDS
+  static constexpr int kSz = kSzLds ? kGU * 1280 : 0;     // 256 rows x (4 + 1) bytes a group
+  // row sums, in whole 64-lane copies (a copy's last lanes may hold nothing)
+  static constexpr int kXs = BF ? (kGU * kRows * 4 + 255) / 256 * 256 : 0;
+  static constexpr int kW = 2 * kX;                       // offset of the codes
+  static constexpr int kS = kW + 4 * 4096;                // offset of the s/z slots
+  static constexpr int kR = kS + 2 * kSz;                 // offset of the row-sum slots
+  static constexpr int kGroup = kR + 2 * kXs;             // LDS of one four-wave group
+  static_assert(kGroup <= 80 * 1024, "two groups fit the LDS of a CU");
+};
 
-__global__ __launch_bounds__(kBWaves * 64, 1) void w4a16_bgemm_kernel(BgemmArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+// Buffer descriptor in SGPRs (untyped dwords, no swizzle) for the copies
+// below.
+PMI_DEV u32x4 descriptor(const void* p, uint32_t bytes) {
+  const uint64_t a = (uint64_t)p;
+  u32x4 d = {(uint32_t)a, (uint32_t)(a >> 32) & 0xFFFFu, bytes, 0x00020000u};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) d[i] = __builtin_amdgcn_readfirstlane(d[i]);
+  return d;
+}
+
+// 16 (or 4) bytes per lane from a buffer to LDS address base + 16 (4) * lane.
+// base is uniform. No register is written; the caller waits with wait_vmcnt<0>.
+PMI_DEV void dma16(u32x4 r, uint32_t base, int voff, int soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(base),
+               "v"(voff), "s"(r), "s"(__builtin_amdgcn_readfirstlane(soff))
+               : "memory");
+#else
+  (void)r, (void)base, (void)voff, (void)soff;
+#endif
+}
+PMI_DEV void dma4(u32x4 r, uint32_t base, int voff, int soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(base),
+               "v"(voff), "s"(r), "s"(__builtin_amdgcn_readfirstlane(soff))
+               : "memory");
+#else
+  (void)r, (void)base, (void)voff, (void)soff;
+#endif
+}
+
+template <bool BF>
+PMI_DEV f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (BF)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+// Rows m .. m + 3 (v[j][e]: row m + e, column row0 + j) to y.
+template <bool BF>
+PMI_DEV void store_rows(uint16_t* __restrict__ y, const f32x4* v, int m, int M, int N, int row0) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (m + e >= M) continue;
+    u32x2 o;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      uint32_t v0, v1;
+      if constexpr (BF) {
+        v0 = f32_to_bf16_rne(v[2 * q][e]);
+        v1 = f32_to_bf16_rne(v[2 * q + 1][e]);
+      } else {
+        v0 = __builtin_bit_cast(uint16_t, f32_to_f16_rne(v[2 * q][e]));
+        v1 = __builtin_bit_cast(uint16_t, f32_to_f16_rne(v[2 * q + 1][e]));
+      }
+      o[q] = v0 | (v1 << 16);
+    }
+    *reinterpret_cast<u32x2*>(y + (size_t)(m + e) * N + row0) = o;
+  }
+}
+
+template <int MT, int KSG, bool BF, int KG, bool RM>
+__global__ __launch_bounds__(256 * KG, 2) void w4a16_bgemm_kernel(BgemmArgs a) {
+  using S = Shape<MT, KSG, BF>;
+  constexpr int GU = S::kGU;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_all[];
 
   const int tid = threadIdx.x, l = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // workgroup 8 k + x -> pair L = x chunk + k of XCD x's range; L runs band
-  // fastest, so an XCD holds consecutive bands of an activation block
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kgrp = KG == 1 ? 0 : wave >> 2, wv = wave & 3;
+  // Workgroup 8 k + x runs on XCD x and takes entry x chunk + k of the list
+  // (activation block, split, band), band fastest: the bands that share
+  // activation rows share an XCD's L2. A placement preference only.
   const int x8 = blockIdx.x % 8, k8 = blockIdx.x / 8;
   const int L = x8 * a.chunk + k8;
-  if (k8 >= a.chunk || L >= a.n_bands * a.grid_m) return;  // padding workgroups (uniform)
-  const int band = L % a.n_bands, mb = L / a.n_bands;
+  if (k8 >= a.chunk || L >= a.n_bands * a.splits * a.grid_m) return;  // padding (uniform)
+  const int band = L % a.n_bands, rest = L / a.n_bands;
+  const int sp = rest % a.splits, mb = rest / a.splits;
   const int M = a.M, N = a.N, K = a.K;
   const int U = K >> 7;
-  const int G = K / a.gs;
-  const int upg = a.gs >> 7;  // units per group
-  const int m0 = 128 * mb;
-  const int ln = l & 15, h = l >> 4;
+  const int u_lo = (int)((int64_t)U * sp / a.splits), u_hi = (int)((int64_t)U * (sp + 1) / a.splits);
+  const int m0 = S::kRows * mb;
+  const int p = band * 4 + wv;
+  const int pc = p < a.n_panels ? p : a.n_panels - 1;
 
-  // ---- staging: wave w moves activation pieces 4 w .. 4 w + 3 (rows 16 w ..
-  // 16 w + 15; lane l: chunk l % 16 of row 4 g + l / 16, read from activation
-  // chunk (l % 16) ^ (row % 16)), weight pieces 2 w, 2 w + 1 (panel i / 4, 1 KiB
-  // piece i % 4; panels past the last read past the buffer's end, where the
-  // buffer resource returns zeros), and wave 0 the band's scales, wave 1 its
-  // zero points
-  const __amdgpu_buffer_rsrc_t rx = rsrc(a.x, (int64_t)M * K * 2);
-  const __amdgpu_buffer_rsrc_t rw = rsrc(a.wt, (int64_t)a.n_panels * 64 * (K >> 1));
-  const __amdgpu_buffer_rsrc_t rs = rsrc(a.s_gm, (int64_t)G * N * 4);
-  const __amdgpu_buffer_rsrc_t rz = rsrc(a.z_gm, (int64_t)G * N);
-  int vx[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = 16 * wv + 4 * i + (l >> 4);
-    const int mg = m0 + row < M ? m0 + row : M - 1;
-    vx[i] = mg * K * 2 + 16 * ((l & 15) ^ (row & 15));
-  }
-  int vwp[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int pc = 2 * wv + i;
-    vwp[i] = (band * 4 + pc / 4) * U * 4096 + (pc % 4) * 1024 + 16 * l;
-  }
-  const int vsz = wv == 0 ? (256 * band + 4 * l) * 4 : 256 * band + 4 * l;
-  // The activation rows are staged two units ahead, in two register stages;
-  // the codes, scales and zero points one unit ahead.
-  struct XStage {
-    u32x4 x[4];
-  };
-  struct WStage {
-    u32x4 w[2], sz;
-  };
-  auto clamp_unit = [&](int u) {
-    u = u < U ? u : U - 1;  // past K: re-read the last unit (never used)
-    return __builtin_amdgcn_readfirstlane(u);
-  };
-  auto load_x = [&](XStage& st, int u) {
-    const int uu = clamp_unit(u);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      st.x[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, vx[i], uu * 256, 0));
-  };
-  auto load_w = [&](WStage& st, int u) {
-    const int uu = clamp_unit(u);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      st.w[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, vwp[i], uu * 4096, 0));
-    const int g = uu / upg;
-    if (wv == 0)
-      st.sz = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, vsz, g * N * 4, 0));
-    else if (wv == 1)
-      st.sz = u32x4{__builtin_amdgcn_raw_buffer_load_b32(rz, vsz, g * N, 0), 0u, 0u, 0u};
-  };
-  auto stage_write = [&](const XStage& xs, const WStage& ws, uint8_t* base) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(base + (4 * wv + i) * 1024 + 16 * l) = xs.x[i];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(base + kBWo + (2 * wv + i) * 1024 + 16 * l) = ws.w[i];
-    if (wv == 0) *reinterpret_cast<u32x4*>(base + kBSo + 16 * l) = ws.sz;
-    else if (wv == 1) *reinterpret_cast<uint32_t*>(base + kBZo + 4 * l) = ws.sz[0];
-  };
+  uint8_t* lds = lds_all + kgrp * S::kGroup;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  // Rows past M lie past the descriptor's end and read as zeros.
+  const int rows = M - m0 < S::kRows ? M - m0 : S::kRows;
+  const u32x4 dx = descriptor(a.x + (int64_t)m0 * K, (uint32_t)rows * K * 2);
+  const u32x4 dw = descriptor(a.w, RM ? (uint32_t)N * (K >> 1) : (uint32_t)a.n_panels * 64 * (K >> 1));
+  const int groups = K / a.gs;
+  const u32x4 ds = descriptor(a.s_gm, (uint32_t)groups * N * 4);
+  const u32x4 dz = descriptor(a.z_gm, (uint32_t)groups * N);
+  const __amdgpu_buffer_rsrc_t rs = rsrc(a.s_gm, (int64_t)groups * N * 4);
+  const __amdgpu_buffer_rsrc_t rz = rsrc(a.z_gm, (int64_t)groups * N);
 
-  // ---- compute: tiles 2 jh, 2 jh + 1 of panel pw, all 128 activation rows
-  const int pw = wv >> 1, jh = wv & 1;
-  const int p = band * 4 + pw;
-  const int row0 = 64 * p + 4 * ln + 2 * jh;
-  f32x4 acc[kBMT][2];
+  // Lane values that a unit needs once are worked out there, from an opaque
+  // copy of the lane id: kept across the MFMAs they would spill.
+  auto lane = [&]() {
+    int v = l;
+    asm volatile("" : "+v"(v));
+    return v;
+  };
+  // Unit u (its first scale group: g) to slot b.
+  auto copy_x = [&](int u, int b) {
+    const int q = lane();
+    const int row0 = 4 * MT * wv + (q >> 4);
+    // chunk (q % 16) ^ (row % 16) of row row0 + 4 i
+    const int r4 = (4 * MT * wv) & 15;
+    const int base = row0 * K * 2;
 #pragma unroll
-  for (int mt = 0; mt < kBMT; ++mt)
+    for (int i = 0; i < MT; ++i)
+      dma16(dx, lds0 + b * S::kX + (wv * MT + i) * 1024,
+            base + i * 8 * K + ((((q & 15) ^ (q >> 4)) << 4) ^ (((r4 + 4 * i) & 12) << 4)), u * 256);
+  };
+  auto copy_w = [&](int u) {
+    const int q = lane();
+    const uint32_t base = lds0 + S::kW + wv * 4096;
+    if constexpr (RM) {
+      // tile j: 16-byte chunk c of row 4 n + j at (16 c + n) * 16
+      int r0 = 64 * p + 4 * (q & 15);
+      r0 = r0 < N ? r0 : N - 4;
+      const int v = r0 * (K >> 1) + 16 * (q >> 4);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto compute = [&](const uint8_t* base) {
-    u32x4 w[2];
+      for (int j = 0; j < 4; ++j) dma16(dw, base + j * 1024, v + j * (K >> 1), u * 64);
+    } else {
+      const int so = (pc * U + u) * 4096;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-      w[j] = *reinterpret_cast<const u32x4*>(base + kBWo + pw * 4096 + (2 * jh + j) * 1024 + 16 * l);
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    const f32x2 sc = *reinterpret_cast<const f32x2*>(base + kBSo + (64 * pw + 4 * ln + 2 * jh) * 4);
-    const uint32_t zq = *reinterpret_cast<const uint16_t*>(base + kBZo + 64 * pw + 4 * ln + 2 * jh);
-    f16x2 nz[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) nz[j] = as_f16x2(neg_magic_zero_x2((zq >> (8 * j)) & 0xFFu));
-    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    f32x4 cg[kBMT][2];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int run = t >> 1, half = t & 1;
-      // the step's two B operands, then each activation tile read once for both
-      f16x8 B[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const uint32_t w0 = w[j][2 * half], w1 = w[j][2 * half + 1];
-        const uint32_t t0 = (run ? (w0 >> 4) : w0) & 0x0F0F0F0Fu;
-        const uint32_t t1 = (run ? (w1 >> 4) : w1) & 0x0F0F0F0Fu;
-        B[j] = b_operand(t0, t1, nz[j]);
-      }
-#pragma unroll
-      for (int i = 0; i < kBMT; ++i) {
-        const f16x8 A = *reinterpret_cast<const f16x8*>(base + (16 * i + ln) * 256 + (((4 * t + h) ^ ln) << 4));
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          cg[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[j], t == 0 ? zero4 : cg[i][j], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < 4; ++j) dma16(dw, base + j * 1024, 16 * q, so + j * 1024);
     }
+  };
+  // Scales and zero points of the band's 256 rows, wave w the unit's group w,
+  // and the rows' sums (BF).
+  auto copy_sz = [&](int u, int g, int b) {
+    if constexpr (S::kSzLds) {
+      const int q = lane();
+      if (wv < GU) {
+        int r0 = 256 * band + 4 * q;
+        r0 = r0 < N ? r0 : N - 4;
+        const uint32_t base = lds0 + S::kS + b * S::kSz + wv * 1280;
+        dma16(ds, base, r0 * 4, (g + wv) * N * 4);
+        dma4(dz, base + 1024, r0, (g + wv) * N);
+      }
+      if constexpr (BF) {
+        constexpr int n = GU * S::kRows;  // floats: GU runs of kRows, at most two per lane of a group
+        const u32x4 dr = descriptor(a.sums + (int64_t)u * GU * a.sums_ld, (uint32_t)GU * a.sums_ld * 4);
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < kBMT; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][j][e] = fmaf(sc[j], cg[i][j][e], acc[i][j][e]);
+        for (int k = 0; k < (n + 255) / 256; ++k) {
+          const int f0 = (4 * k + wv) * 64;  // this wave's first float
+          if (f0 < n) {
+            int f = f0 + q;
+            f = f < n ? f : n - 1;
+            const int gg = f / S::kRows;
+            dma4(dr, lds0 + S::kR + b * S::kXs + f0 * 4, (gg * a.sums_ld + m0 + f - gg * S::kRows) * 4, 0);
+          }
+        }
+      }
+    }
+  };
+  f32x4 s_next = {};  // fp16, group sizes of 128 and more: the next unit's
+  uint32_t z_next = 0;
+  auto load_sz = [&](int g) {
+    if constexpr (!S::kSzLds) {
+      int r0 = 64 * p + 4 * (lane() & 15);
+      r0 = r0 < N ? r0 : N - 4;
+      s_next = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, r0 * 4, g * N * 4, 0));
+      z_next = __builtin_amdgcn_raw_buffer_load_b32(rz, r0, g * N, 0);
+    }
   };
 
-  // Unit u: activations in xs[u % 2] (loaded during unit u - 2), codes in ws
-  // (loaded during unit u - 1). Issue order within a step is codes, then
-  // activations, so the wait for the codes leaves the younger activations in
-  // flight.
-  XStage xs[2];
-  WStage ws;
-  load_x(xs[0], 0);
-  load_w(ws, 0);
-  stage_write(xs[0], ws, lds);
-  load_x(xs[1], 1);
-  load_w(ws, 1);
-  load_x(xs[0], 2);
-  wait_lgkm0();
-  barrier_only();
-  // step s: compute unit s, write unit s + 1 to the other slot (whose unit
-  // s - 1 every wave finished before the last barrier), fetch the codes of
-  // s + 2 and the activations of s + 3
-  auto step = [&](int s, XStage& x1) {
-    compute(lds + (s & 1) * kBSlot);
-    __builtin_amdgcn_sched_barrier(0);
-    stage_write(x1, ws, lds + ((s + 1) & 1) * kBSlot);
-    load_w(ws, s + 2);
-    load_x(x1, s + 3);
-    // the slot writes have landed before any wave passes (LDS operations
-    // complete in order per wave; the barrier makes them visible)
-    wait_lgkm0();
+  f32x4 acc[MT][4];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+
+  // group of unit u: u / units-per-group, stepped without a division
+  const int upg = KSG == 4 ? a.gs >> 7 : 1;
+  int u = u_lo + kgrp, g, ug;
+  if constexpr (KSG == 4) {
+    g = u / upg;
+    ug = u - g * upg;
+  } else {
+    g = GU * u;
+    ug = 0;
+  }
+  {
+    const bool in = u < u_hi;
+    load_sz(in ? g : 0);
+    if (in) {
+      copy_w(u);
+      copy_sz(u, g, 0);
+      copy_x(u, 0);
+    }
+  }
+  const int steps = (u_hi - u_lo + KG - 1) / KG;  // the same for both groups: they share the barriers
+  for (int s = 0; s < steps; ++s, u += KG) {
+    wait_vmcnt<0>();
     barrier_only();
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // whole pairs of steps with no exit inside, then the last two units (U is
-  // even and at least 12: K % 512 == 0, K >= 1536)
-  int s = 0;
-  for (; s < U - 2; s += 2) {
-    step(s, xs[1]);
-    step(s + 1, xs[0]);
-  }
-  step(U - 2, xs[1]);
-  compute(lds + ((U - 1) & 1) * kBSlot);
-  if (p >= a.n_panels || row0 >= N) return;
+    const int slot = s & 1;
+    if (KG > 1 && u >= u_hi) continue;  // the shorter group's last step (uniform per wave)
 
-  // lane (n, h): activation rows m0 + 16 i + 4 h + e, weight rows row0 + j
+    // codes to registers; their LDS and the other slots may then be refilled
+    const uint8_t* wb = lds + S::kW + wv * 4096;
+    u32x4 w[4];
+    u32x2 w32[4][4];  // RM, 32-column groups: one 8-byte piece per k-step
+    {
+      const int q = lane();
+      if constexpr (RM && KSG == 1) {
 #pragma unroll
-  for (int i = 0; i < kBMT; ++i)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int m = m0 + 16 * i + 4 * h + e;
-      if (m >= M) continue;
-      const uint32_t v0 = __builtin_bit_cast(uint16_t, f32_to_f16_rne(acc[i][0][e]));
-      const uint32_t v1 = __builtin_bit_cast(uint16_t, f32_to_f16_rne(acc[i][1][e]));
-      *reinterpret_cast<uint32_t*>(a.y + (size_t)m * N + row0) = v0 | (v1 << 16);
+          for (int t = 0; t < 4; ++t)
+            w32[j][t] = *reinterpret_cast<const u32x2*>(wb + j * 1024 + t * 256 + 16 * (q & 15) + 8 * ((q >> 4) & 1));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(w32[j][0]), "+v"(w32[j][1]), "+v"(w32[j][2]), "+v"(w32[j][3])::"memory");
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (RM) {
+            const int o = j * 1024 + 256 * (q >> 5) + 16 * (q & 15) + 8 * ((q >> 4) & 1);
+            const u32x2 lo = *reinterpret_cast<const u32x2*>(wb + o);
+            const u32x2 hi = *reinterpret_cast<const u32x2*>(wb + o + 512);
+            w[j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+          } else {
+            w[j] = *reinterpret_cast<const u32x4*>(wb + j * 1024 + 16 * q);
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3])::"memory");
+      }
     }
+    f32x4 sc[GU];
+    uint32_t zq[GU];
+    if constexpr (S::kSzLds) {
+      const int q = lane();
+      const uint8_t* sb = lds + S::kS + slot * S::kSz + 256 * wv + 16 * (q & 15);
+      const uint8_t* zb = lds + S::kS + slot * S::kSz + 1024 + 64 * wv + 4 * (q & 15);
+#pragma unroll
+      for (int gg = 0; gg < GU; ++gg) {
+        sc[gg] = *reinterpret_cast<const f32x4*>(sb + gg * 1280);
+        zq[gg] = *reinterpret_cast<const uint32_t*>(zb + gg * 1280);
+      }
+    } else {
+      sc[0] = s_next;
+      zq[0] = z_next;
+    }
+    const bool more = u + KG < u_hi;
+    if constexpr (KSG == 4) {
+#pragma unroll
+      for (int n = 0; n < KG; ++n)
+        if (++ug == upg) ug = 0, ++g;
+    } else {
+      g += GU * KG;
+    }
+    load_sz(more ? g : 0);
+    if (more) {
+      copy_w(u + KG);
+      copy_sz(u + KG, g, slot ^ 1);
+      copy_x(u + KG, slot ^ 1);
+    }
+
+    // A operand of k-step t: row n of each tile, chunk (4 t + h) ^ n
+    int ao[4];
+    {
+      const int q = lane();
+      const int o = ((q & 15) << 8) + (((q & 15) ^ (q >> 4)) << 4);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ao[t] = o ^ (64 * t);
+    }
+    const uint8_t* xb = lds + slot * S::kX;
+    u32x4 A[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) A[t] = *reinterpret_cast<const u32x4*>(xb + ao[t]);
+    f32x4 xs[BF ? GU : 1];
+    const uint8_t* rb = lds + S::kR + slot * S::kXs;
+    int ro = 0;
+    if constexpr (BF) {
+      ro = (lane() >> 4) << 4;
+#pragma unroll
+      for (int gg = 0; gg < GU; ++gg) xs[gg] = *reinterpret_cast<const f32x4*>(rb + ro + gg * S::kRows * 4);
+    }
+
+    u32x4 B[4][4];
+    float zf[GU][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint32_t z = (zq[t / KSG] >> (8 * j)) & 0xFFu;
+        uint32_t w0, w1;
+        if constexpr (RM && KSG == 1) {
+          const int sh = 4 * (lane() >> 5);
+          w0 = w32[j][t][0] >> sh, w1 = w32[j][t][1] >> sh;
+        } else {
+          // tiled and 128-column groups: k-steps (0, 1) low nibbles, (2, 3) high;
+          // row-major 64-column groups: low and high nibbles alternate
+          const int piece = RM && KSG == 2 ? t >> 1 : t & 1, high = RM && KSG == 2 ? t & 1 : t >> 1;
+          w0 = w[j][2 * piece], w1 = w[j][2 * piece + 1];
+          if (high) w0 >>= 4, w1 >>= 4;
+        }
+        w0 &= 0x0F0F0F0Fu, w1 &= 0x0F0F0F0Fu;
+        if constexpr (BF) {
+          B[j][t] = __builtin_bit_cast(u32x4, b_operand_bf16(w0, w1));
+          if (t % KSG == 0) zf[t / KSG][j] = -(128.f + (float)z);
+        } else {
+          B[j][t] = __builtin_bit_cast(u32x4, b_operand(w0, w1, as_f16x2(neg_magic_zero_x2(z))));
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+    // step (i, q, gg): activation tile i, weight tiles 2 q and 2 q + 1, scale group gg
+    f32x4 cg[2][2];
+    int pi = 0, pq = 0, pg = 0;  // the step whose fold is pending
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+#pragma unroll
+        for (int gg = 0; gg < GU; ++gg) {
+          const int buf = ((2 * i + q) * GU + gg) & 1;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            if constexpr (BF) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) cg[buf][j][e] = xs[gg][e] * zf[gg][2 * q + j];
+            }
+          }
+          if (BF && q == 1 && i + 1 < MT)
+            xs[gg] = *reinterpret_cast<const f32x4*>(rb + ro + (gg * S::kRows + 16 * (i + 1)) * 4);
+#pragma unroll
+          for (int t = gg * KSG; t < (gg + 1) * KSG; ++t) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              cg[buf][j] = mfma<BF>(A[t], B[2 * q + j][t], !BF && t == gg * KSG ? zero4 : cg[buf][j]);
+            if (q == 1 && i + 1 < MT) A[t] = *reinterpret_cast<const u32x4*>(xb + ao[t] + (i + 1) * 4096);
+          }
+          if (i + q + gg > 0) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                acc[pi][2 * pq + j][e] = fmaf(sc[pg][2 * pq + j], cg[buf ^ 1][j][e], acc[pi][2 * pq + j][e]);
+          }
+          pi = i, pq = q, pg = gg;
+          // MFMAs first (the pending sums' last ones are still in flight), then
+          // two folds to each
+          if constexpr (KSG == 4 && !BF) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 3, 0);
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+              __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+              __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+              if (q) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[MT - 1][2 + j][e] = fmaf(sc[GU - 1][2 + j], cg[(2 * MT * GU - 1) & 1][j][e], acc[MT - 1][2 + j][e]);
+    __builtin_amdgcn_s_setprio(0);
+  }
+
+  const int t256 = tid & 255;
+  constexpr int H = KG == 1 ? MT : (MT + 1) / 2;  // activation tiles that group 0 finishes
+  if constexpr (KG == 2) {
+    // each group hands the other the tiles that one finishes
+    __syncthreads();
+    f32x4* ex = reinterpret_cast<f32x4*>(lds_all);
+    if (kgrp == 1) {
+#pragma unroll
+      for (int i = 0; i < H; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ex[(4 * i + j) * 256 + t256] = acc[i][j];
+    } else {
+#pragma unroll
+      for (int i = H; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ex[(4 * i + j) * 256 + t256] = acc[i][j];
+    }
+    __syncthreads();
+    if (kgrp == 0) {
+#pragma unroll
+      for (int i = 0; i < H; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] += ex[(4 * i + j) * 256 + t256];
+    } else {
+#pragma unroll
+      for (int i = H; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] += ex[(4 * i + j) * 256 + t256];
+    }
+  }
+
+  if (a.splits > 1) {
+    // partial tile of split sp: [4 i + j][thread] x 16 bytes, for the combine
+    float* part = a.part + ((size_t)(mb * a.n_bands + band) * a.splits + sp) * (MT * 4 * 256 * 4);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      if (KG == 2 && (i < H) != (kgrp == 0)) continue;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) reinterpret_cast<f32x4*>(part)[(4 * i + j) * 256 + t256] = acc[i][j];
+    }
+    return;
+  }
+
+  // lane (n, h): activation rows m0 + 16 i + 4 h + e, weight rows row0 .. row0 + 3
+  const int row0 = 64 * p + 4 * (l & 15);
+  if (p >= a.n_panels || row0 >= N) return;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    if (KG == 2 && (i < H) != (kgrp == 0)) continue;
+    store_rows<BF>(a.y, acc[i], m0 + 16 * i + 4 * (l >> 4), M, N, row0);
+  }
 }
 
-}  // namespace
-
-BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs) {
-  BgemmConfig c{};
-  c.ok = false;
-  if (M < 1 || N % 4 != 0 || K % 128 != 0 || K < 128 || gs % 128 != 0 || K % gs != 0) return c;
-  if ((int64_t)M * K * 2 >= (1ll << 31) || ((N + 63) / 64) * 64 * (K / 2) >= (1ll << 31)) return c;
-  const int64_t bands = ((N + 63) / 64 + 3) / 4;
-  const int64_t gm = (M + 127) / 128;
-  const int64_t chunk = (bands * gm + 7) / 8;
-  if (8 * chunk >= (1ll << 31)) return c;
-  c.ok = true;
-  c.n_bands = (int)bands;
-  c.grid_m = (int)gm;
-  c.chunk = (int)chunk;
-  c.grid = (int)(8 * chunk);
-  return c;
+// Split K: y = the partial tiles added in split order, one thread per four
+// activation rows x four weight rows. A launch of its own: the last workgroup
+// of a tile adding them alone read up to 1 MiB by itself (8 splits: 27 us for
+// 1024 x 4096 at M = 128, of which the products are a quarter).
+template <int MT, bool BF>
+__global__ __launch_bounds__(256) void bgemm_combine_kernel(const float* __restrict__ part,
+                                                            uint16_t* __restrict__ y, int M, int N,
+                                                            int n_bands, int splits) {
+  const int t = threadIdx.x, l = t & 63;
+  const int i = blockIdx.x % MT, tl = blockIdx.x / MT;
+  const int band = tl % n_bands, mb = tl / n_bands;
+  const int row0 = 256 * band + 64 * (t >> 6) + 4 * (l & 15);
+  const int m = 16 * (MT * mb + i) + 4 * (l >> 4);
+  if (row0 >= N || m >= M) return;
+  constexpr int kPart = MT * 4 * 256;  // f32x4 per partial tile
+  const f32x4* src = reinterpret_cast<const f32x4*>(part) + (size_t)tl * splits * kPart + 4 * i * 256 + t;
+  f32x4 v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = src[j * 256];
+  for (int q = 1; q < splits; ++q)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] += src[(size_t)q * kPart + j * 256];
+  store_rows<BF>(y, v, m, M, N, row0);
 }
 
-hipError_t launch_bgemm(const void* x, const uint8_t* w_tiled, const float* scales_gm,
-                        const uint8_t* zeros_gm, void* y, int64_t M, int64_t N, int64_t K, int64_t gs,
-                        hipStream_t stream) {
-  const BgemmConfig c = bgemm_config(M, N, K, gs);
-  if (!c.ok) return hipErrorInvalidValue;
+// sums[k / cols][m] = sum of the bf16 row x[m] over columns k .. k + cols - 1
+// (cols 32, 64 or 128), one wave per row, 8 columns per lane and step.
+__global__ __launch_bounds__(256) void bgemm_row_sums_kernel(const uint16_t* __restrict__ x,
+                                                             float* __restrict__ sums, int M, int K,
+                                                             int lanes, int ld) {
+  const int l = threadIdx.x & 63, m = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (m >= M) return;
+  const int chunks = K >> 3;
+  for (int c = l; c < ((chunks + 63) & ~63); c += 64) {
+    float v = 0.f;
+    if (c < chunks) {
+      const u32x4 d = *reinterpret_cast<const u32x4*>(x + (int64_t)m * K + 8 * c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v += __builtin_bit_cast(float, d[i] << 16) + __builtin_bit_cast(float, d[i] & 0xFFFF0000u);
+    }
+    for (int o = lanes >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if (c < chunks && l % lanes == 0) sums[(int64_t)(c / lanes) * ld + m] = v;
+  }
+}
+
+template <int MT, int KSG, bool BF, int KG, bool RM>
+hipError_t launch_one(const BgemmArgs& a, int grid, size_t lds, hipStream_t stream) {
   static std::atomic<uint64_t> allowed{0};
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
   const uint64_t bit = 1ull << (dev & 63);
-  const size_t lds = 2 * (size_t)kBSlot;
+  const void* fn = reinterpret_cast<const void*>(&w4a16_bgemm_kernel<MT, KSG, BF, KG, RM>);
   if (!(allowed.load() & bit)) {
-    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&w4a16_bgemm_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         e != hipSuccess)
       return e;
     allowed.fetch_or(bit);
   }
-  BgemmArgs a;
-  a.x = (const f16*)x;
-  a.wt = w_tiled;
+  hipLaunchKernelGGL((w4a16_bgemm_kernel<MT, KSG, BF, KG, RM>), dim3(grid), dim3(256 * KG), lds, stream, a);
+  return hipGetLastError();
+}
+
+template <int MT, int KSG, bool BF>
+hipError_t launch_shape(const BgemmArgs& a, const BgemmConfig& c, bool rm, hipStream_t stream) {
+  const size_t lds = (size_t)c.kg * Shape<MT, KSG, BF>::kGroup;
+  hipError_t e;
+  if (c.kg == 2)
+    e = rm ? launch_one<MT, KSG, BF, 2, true>(a, c.grid, lds, stream)
+           : launch_one<MT, KSG, BF, 2, false>(a, c.grid, lds, stream);
+  else
+    e = rm ? launch_one<MT, KSG, BF, 1, true>(a, c.grid, lds, stream)
+           : launch_one<MT, KSG, BF, 1, false>(a, c.grid, lds, stream);
+  if (e != hipSuccess || a.splits == 1) return e;
+  hipLaunchKernelGGL((bgemm_combine_kernel<MT, BF>), dim3(MT * a.n_bands * a.grid_m), dim3(256), 0, stream,
+                     a.part, a.y, a.M, a.N, a.n_bands, a.splits);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16) {
+  BgemmConfig c{};
+  c.ok = false;
+  if (M < 1 || N < 4 || N % 4 != 0 || K % 128 != 0 || K < 128 || K % gs != 0) return c;
+  if (gs != 32 && gs != 64 && gs % 128 != 0) return c;
+  if (M * K * 2 >= (1ll << 31) || ((N + 63) / 64) * 64 * (K / 2) >= (1ll << 31)) return c;
+  c.mt = gs == 32 ? 6 : (gs == 64 || bf16) ? 7 : 8;
+  const int64_t bands = ((N + 63) / 64 + 3) / 4;
+  const int64_t gm = (M + 16 * c.mt - 1) / (16 * c.mt);
+  const int64_t cus = device_cu_count(), tiles = bands * gm, units = K / 128;
+  c.n_bands = (int)bands;
+  c.grid_m = (int)gm;
+  // One workgroup of two groups per CU up to one tile per CU; past that two
+  // workgroups of one group.
+  c.kg = tiles <= cus && units > 1 ? 2 : 1;
+  // Fewer tiles than half the CUs: split K, at least kMinUnits units a split.
+#ifndef KMINU
+#define KMINU 4
+#endif
+  constexpr int kMinUnits = KMINU;
+  int64_t splits = 1;
+  if (2 * tiles <= cus) {
+    splits = cus / tiles;
+    if (splits > units / kMinUnits) splits = units / kMinUnits;
+    if (splits > 16) splits = 16;
+    if (splits < 1) splits = 1;
+  }
+  c.splits = (int)splits;
+  c.ws_split = splits > 1 ? (size_t)tiles * splits * c.mt * 4 * 256 * 16 : 0;
+  c.sums_ld = (int)(gm * 16 * c.mt);
+  c.ws_sums = bf16 ? ws_align((size_t)(K / (gs < 128 ? gs : 128)) * c.sums_ld * 4) : 0;
+  const int64_t chunk = (tiles * splits + 7) / 8;
+  if (8 * chunk >= (1ll << 31)) return c;
+  c.chunk = (int)chunk;
+  c.grid = (int)(8 * chunk);
+  c.ok = true;
+  return c;
+}
+
+hipError_t launch_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w_kernel, const float* scales_gm,
+                        const uint8_t* zeros_gm, void* y, int64_t M, int64_t N, int64_t K, int64_t gs,
+                        bool bf16, void* workspace, size_t ws_bytes, size_t ws_offset, hipStream_t stream) {
+  BgemmConfig c = bgemm_config(M, N, K, gs, bf16);
+  if (!c.ok) return hipErrorInvalidValue;
+  BgemmArgs a{};
+  size_t off = ws_offset;
+  if (bf16) {
+    if (!workspace || ws_bytes < off + c.ws_sums) return hipErrorInvalidValue;
+    float* sums = (float*)((uint8_t*)workspace + off);
+    off += c.ws_sums;
+    hipLaunchKernelGGL(bgemm_row_sums_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, stream,
+                       (const uint16_t*)x, sums, (int)M, (int)K, (int)((gs < 128 ? gs : 128) / 8), c.sums_ld);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    a.sums = sums;
+  }
+  if (c.splits > 1 && (!workspace || ws_bytes < off + c.ws_split)) {
+    c.splits = 1;  // no room for the partial tiles
+    c.chunk = (c.n_bands * c.grid_m + 7) / 8;
+    c.grid = 8 * c.chunk;
+  }
+  const bool rm = w_tiled == nullptr;
+  a.x = (const uint16_t*)x;
+  a.w = rm ? w_kernel : w_tiled;
   a.s_gm = scales_gm;
   a.z_gm = zeros_gm;
-  a.y = (f16*)y;
+  a.y = (uint16_t*)y;
+  a.part = (float*)((uint8_t*)workspace + off);
   a.M = (int)M;
   a.N = (int)N;
   a.K = (int)K;
@@ -304,9 +675,14 @@ hipError_t launch_bgemm(const void* x, const uint8_t* w_tiled, const float* scal
   a.n_panels = (int)((N + 63) / 64);
   a.n_bands = c.n_bands;
   a.grid_m = c.grid_m;
+  a.splits = c.splits;
   a.chunk = c.chunk;
-  hipLaunchKernelGGL(w4a16_bgemm_kernel, dim3(c.grid), dim3(kBWaves * 64), lds, stream, a);
-  return hipGetLastError();
+  a.sums_ld = c.sums_ld;
+  if (gs == 32)
+    return bf16 ? launch_shape<6, 1, true>(a, c, rm, stream) : launch_shape<6, 1, false>(a, c, rm, stream);
+  if (gs == 64)
+    return bf16 ? launch_shape<7, 2, true>(a, c, rm, stream) : launch_shape<7, 2, false>(a, c, rm, stream);
+  return bf16 ? launch_shape<7, 4, true>(a, c, rm, stream) : launch_shape<8, 4, false>(a, c, rm, stream);
 }
 
 }  // namespace pmi

@@ -81,29 +81,46 @@ __global__ void perm_u16_kernel(const int32_t* __restrict__ perm, uint16_t* __re
   if (bad && local_bad) atomicAdd(bad, local_bad);
 }
 
-// [N, G] -> [G, N] copies of the scales and zero points (zeros to u8, values
-// that are not integers in [0, 15] counted like zeros_to_u8_kernel). One
-// thread per output element: writes are coalesced, reads strided; it runs
-// once per layer.
-__global__ void sz_group_major_kernel(const float* __restrict__ scales,
-                                      const void* __restrict__ zeros, int zero_u8,
-                                      float* __restrict__ s_gm, uint8_t* __restrict__ z_gm,
-                                      int32_t* __restrict__ bad, int64_t N, int64_t G) {
+// [N, G] -> [G, N] copies of the scales and zero points. strict: zeros that are
+// not integers in [0, 15] become 0 and are counted like zeros_to_u8_kernel;
+// otherwise they are converted as the matmul kernels convert them. A workgroup
+// turns 64 rows x 32 groups in LDS, so that reads run along G and writes along
+// N (one thread per output element, reads G apart, took 6.4 us for 14336 x 32;
+// this 3.2).
+__global__ __launch_bounds__(kBlock) void sz_group_major_kernel(
+    const float* __restrict__ scales, const void* __restrict__ zeros, int zero_u8, int strict,
+    float* __restrict__ s_gm, uint8_t* __restrict__ z_gm, int32_t* __restrict__ bad, int64_t N,
+    int64_t G) {
+  __shared__ float st[32][65];
+  __shared__ uint8_t zt[32][68];
+  const int64_t n0 = (int64_t)blockIdx.x * 64;
   int local_bad = 0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N * G;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t g = i / N, n = i - g * N;
-    s_gm[i] = scales[n * G + g];
-    if (zero_u8) {
-      const uint8_t z = ((const uint8_t*)zeros)[n * G + g];
-      local_bad += z <= 15 ? 0 : 1;
-      z_gm[i] = z <= 15 ? z : (uint8_t)0;
-    } else {
-      const float z = ((const float*)zeros)[n * G + g];
-      const bool ok = z >= 0.f && z <= 15.f && z == rintf(z);  // false for NaN
-      local_bad += ok ? 0 : 1;
-      z_gm[i] = ok ? (uint8_t)(int)z : (uint8_t)0;
+  for (int64_t g0 = (int64_t)blockIdx.y * 32; g0 < G; g0 += (int64_t)gridDim.y * 32) {
+    const int gi = threadIdx.x & 31;
+    for (int r = threadIdx.x >> 5; r < 64; r += kBlock / 32) {
+      if (n0 + r >= N || g0 + gi >= G) continue;
+      const int64_t i = (n0 + r) * G + g0 + gi;
+      st[gi][r] = scales[i];
+      if (zero_u8) {
+        const uint8_t z = ((const uint8_t*)zeros)[i];
+        const bool ok = z <= 15 || !strict;
+        local_bad += ok ? 0 : 1;
+        zt[gi][r] = ok ? z : (uint8_t)0;
+      } else {
+        const float z = ((const float*)zeros)[i];
+        const bool ok = (z >= 0.f && z <= 15.f && z == rintf(z)) || !strict;  // false for NaN
+        local_bad += ok ? 0 : 1;
+        zt[gi][r] = ok ? (uint8_t)(uint32_t)(int)z : (uint8_t)0;
+      }
     }
+    __syncthreads();
+    const int r = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q < 32; q += kBlock / 64) {
+      if (n0 + r >= N || g0 + q >= G) continue;
+      s_gm[(g0 + q) * N + n0 + r] = st[q][r];
+      z_gm[(g0 + q) * N + n0 + r] = zt[q][r];
+    }
+    __syncthreads();
   }
   if (bad && local_bad) atomicAdd(bad, local_bad);
 }
@@ -418,11 +435,12 @@ hipError_t launch_perm_u16(const int32_t* perm, uint16_t* out, int32_t* bad, int
   return hipGetLastError();
 }
 
-hipError_t launch_sz_group_major(const float* scales, const void* zeros, int zero_u8,
+hipError_t launch_sz_group_major(const float* scales, const void* zeros, int zero_u8, int strict,
                                  float* scales_gm, uint8_t* zeros_gm, int32_t* bad, int64_t N,
                                  int64_t G, hipStream_t stream) {
-  hipLaunchKernelGGL(sz_group_major_kernel, dim3(grid_for(N * G)), dim3(kBlock), 0, stream, scales,
-                     zeros, zero_u8, scales_gm, zeros_gm, bad, N, G);
+  const int64_t gy = (G + 31) / 32;
+  hipLaunchKernelGGL(sz_group_major_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)(gy < 65535 ? gy : 65535)),
+                     dim3(kBlock), 0, stream, scales, zeros, zero_u8, strict, scales_gm, zeros_gm, bad, N, G);
   return hipGetLastError();
 }
 

@@ -107,7 +107,10 @@ def _workspace(dev: torch.device, stream: int, nbytes: int) -> torch.Tensor | No
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
-        _WORKSPACES[key] = ws
+        # under capture the zero fill is only recorded: such a workspace belongs
+        # to the graph, whose replays fill it, and is not kept for eager calls
+        if not torch.cuda.is_current_stream_capturing():
+            _WORKSPACES[key] = ws
     return ws
 
 
@@ -233,7 +236,7 @@ def _matmul(x, packed_weight, scales, zeros, group_size, perm, perm16, sz_gm, w_
             f"out must be a contiguous [M, N] {x.dtype} tensor"
     with _DeviceGuard(dev):
         stream = _stream_handle(dev)
-        nbytes = L.pmi_matmul_workspace_bytes(M, N, K, group_size, int(perm is not None))
+        nbytes = L.pmi_matmul_best_workspace_bytes(M, N, K, group_size, int(perm is not None))
         ws = _workspace(dev, stream, nbytes)
         _lib.check(L.pmi_matmul_w4a16(
             xa.data_ptr(), code, w.data_ptr(), s2.data_ptr(), z2.data_ptr(), zdt,

@@ -1,0 +1,155 @@
+"""The big-tile GEMM beyond its fp16, 128-column-group, tiled-copy case (which
+tests/test_tgemm.py covers): group sizes 32 and 64, bf16, callers without the
+tiled or group-major copies, split K, act_order, ragged M, N and K.
+
+Each case runs through the public operator, is compared with a float64 product
+of the oracle's dequantised weights under a bound derived from the arithmetic,
+and with the GEMV (the general path, forced) under twice that bound."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import pare_amd as P
+from oracle import pare_oracle as O
+from pare_amd import _lib
+from pare_amd.kernels import force_kernel
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+COUNTERS = 64 * 1024   # the counter block every workspace starts with
+
+
+def _case(N, K, gs, seed, act_order):
+    w = (torch.randn(N, K, generator=torch.Generator().manual_seed(seed)) * 0.02).numpy()
+    perm = None
+    if act_order:
+        packed, s, z, g_idx = O.rtn_quantize_act_order(
+            w, np.random.default_rng(seed).permutation(K), gs)
+        w_hat = O.dequantize_gidx(O.unpack_int4(packed), s, z, g_idx)
+        perm = P.perm_from_g_idx(torch.from_numpy(g_idx).to(DEV), gs)
+    else:
+        packed, s, z = O.rtn_quantize(w, gs)
+        w_hat = O.dequantize_packed(packed, s, z)
+    wk = P.repack_int4_for_kernel(torch.from_numpy(packed).to(DEV), gs, perm=perm)
+    return wk, torch.from_numpy(s).to(DEV), P.zeros_to_u8(torch.from_numpy(z).to(DEV)), perm, w_hat
+
+
+def _bound(x, w_hat, s, gs, bf16):
+    """Output rounding (half an ulp of 11 or 8 bits) plus the fp32 sums: at most
+    K + G + 4 roundings of 2^-24 of the sum of the terms' sizes, |x| s 15 in fp16
+    and, in bf16, |x| s (143 + 143) for the products with 128 + q and their
+    correction by 128 + z."""
+    K = x.shape[1]
+    scale = np.repeat(s.cpu().numpy().reshape(w_hat.shape[0], -1), gs, axis=1)[:, :K]
+    size = np.abs(x) @ np.abs(scale).T * (286.0 if bf16 else 15.0)
+    ref = x @ w_hat.astype(np.float64).T
+    return ref, np.abs(ref) * 2.0 ** (-8 if bf16 else -11) + size * (K + K // gs + 4) * 2.0 ** -24 + 2.0 ** -25
+
+
+@pytest.mark.parametrize("M,N,K,gs,bf16,copies,act_order", [
+    # gs 64 / 32 on the tiled copy: split K, one tile of rows and its edges, no split
+    (205, 4096, 4096, 64, False, True, False), (224, 3844, 4096, 64, False, True, False),
+    (400, 14300, 1536, 64, False, True, False), (385, 4100, 2048, 32, False, True, False),
+    (90, 2560, 14336, 32, False, True, True),
+    # bf16, every group size, tiled copy and row-major weights
+    (25, 14000, 1536, 128, True, True, False), (113, 4100, 1536, 128, True, True, False),
+    (225, 2060, 2048, 256, True, True, True), (97, 516, 1536, 64, True, True, False),
+    (193, 260, 1536, 32, True, True, False), (112, 772, 384, 128, True, False, False),
+    (130, 516, 1152, 64, True, False, True), (96, 68, 640, 32, True, False, False),
+    (12, 16644, 2048, 128, True, False, False), (640, 14340, 256, 128, True, False, False),
+    # fp16 without the copies: column counts and group sizes only the GEMV reads
+    (25, 260, 384, 128, False, False, False), (60, 1028, 1408, 128, False, False, True),
+    (33, 64, 128, 64, False, False, False), (225, 516, 1152, 64, False, False, False),
+    (97, 900, 160 * 4, 32, False, False, False), (12, 16644, 2048, 32, False, False, True),
+    # fp16 without the copies, large enough to leave the register-streamed GEMM
+    (769, 5636, 4096, 128, False, False, False),
+])
+def test_bgemm_routes_against_fp64_and_the_gemv(M, N, K, gs, bf16, copies, act_order):
+    wk, s, zu8, perm, w_hat = _case(N, K, gs, M + N % 101, act_order)
+    kw = {"perm": perm}
+    if copies:
+        kw.update(sz_gm=P.sz_group_major(s, zu8), w_tiled=P.tile_w4a16(wk, gs))
+    # the workspace that only the big-tile route asks for: more than the counters
+    # and the act_order gather
+    gathered = (M * K * 2 + 255) // 256 * 256 if act_order else 0
+    planned = _lib.lib().pmi_matmul_best_workspace_bytes(M, N, K, gs, int(act_order))
+    print(f"[case] bgemm M={M} N={N} K={K} gs={gs} bf16={bf16} copies={copies} act={act_order} "
+          f"workspace={planned}", flush=True)
+    assert planned > COUNTERS + gathered
+    op = P.matmul_w4a16_bf16 if bf16 else P.matmul_w4a16
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(
+        torch.bfloat16 if bf16 else torch.float16)
+    xd = x.to(DEV)
+    y = op(xd, wk, s, zu8, gs, **kw)
+    y2 = op(xd, wk, s, zu8, gs, **kw)
+    with force_kernel("gemv"):
+        yg = op(xd, wk, s, zu8, gs, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+    # act_order: w_hat is in the original column order, so the scales of a row
+    # are only bounded by their largest
+    if act_order:
+        s = s.reshape(N, -1).amax(1, keepdim=True).expand(N, K // gs)
+    ref, bound = _bound(x.double().numpy(), w_hat, s, gs, bf16)
+    err = np.abs(y.double().cpu().numpy() - ref)
+    assert (err <= bound).all(), f"max {np.max(err / bound):.2f} of the bound"
+    diff = np.abs(y.double().cpu().numpy() - yg.double().cpu().numpy())
+    assert (diff <= 2 * bound).all(), f"against the GEMV: {np.max(diff / bound):.2f} of the bound"
+
+
+def test_bgemm_route_needs_no_workspace_and_no_alignment_of_y():
+    """With no workspace, or a y that is not 8-byte aligned, bf16 calls of many
+    rows run on the GEMV as before, through the C ABI."""
+    M, N, K, gs = 64, 512, 1536, 128
+    wk, s, zu8, _, _ = _case(N, K, gs, 5, False)
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1)).bfloat16()
+    s2 = s.reshape(N, -1).contiguous()
+    L = _lib.lib()
+    buf = torch.zeros(M * N + 4, dtype=torch.bfloat16, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def call(y, ws):
+        return L.pmi_matmul_w4a16(x.data_ptr(), _lib.PMI_BF16, wk.data_ptr(), s2.data_ptr(),
+                                  zu8.data_ptr(), _lib.PMI_U8, None, None, None, None, None,
+                                  y.data_ptr(), _lib.PMI_BF16, M, N, K, gs,
+                                  ws.data_ptr() if ws is not None else None,
+                                  ws.numel() if ws is not None else 0, stream)
+
+    with force_kernel("gemv"):
+        want = P.matmul_w4a16_bf16(x, wk, s, zu8, gs)
+    ws = torch.zeros(L.pmi_matmul_best_workspace_bytes(M, N, K, gs, 0), dtype=torch.uint8, device=DEV)
+    for y, w in ((buf[:M * N], None), (buf[1:M * N + 1], ws)):
+        assert call(y, w) == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(M, N).view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("bf16,gs", [(True, 128), (False, 64)])
+def test_bgemm_in_a_captured_graph(bf16, gs):
+    """A captured call that no eager call warmed up (its workspace then belongs
+    to the graph), replayed with eager work of the same shape in between."""
+    M, N, K = 130, 1028, 1152
+    wk, s, zu8, _, _ = _case(N, K, gs, 9, False)
+    op = P.matmul_w4a16_bf16 if bf16 else P.matmul_w4a16
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(2))
+    x = x.bfloat16() if bf16 else x.half()
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        y = op(x, wk, s, zu8, gs)
+    for k in range(3):
+        x.add_(1.0)
+        want = op(x, wk, s, zu8, gs)
+        with torch.cuda.stream(side):
+            eager = op(x, wk, s, zu8, gs)
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16)), k
+        assert torch.equal(eager.view(torch.int16), want.view(torch.int16)), k
