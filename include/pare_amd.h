@@ -385,6 +385,15 @@ PMI_API int pmi_gptq_group_params(const float* w, int64_t ldw, int64_t N, int64_
                                   int64_t cols, int sym, float* scale, float* zero, int64_t G,
                                   int64_t g, void* stream);
 
+/* Cholesky factor L (a = L L^T) of an n x n diagonal block, n <= 128, of a
+ * row-major fp64 matrix with row stride ld: the lower triangle of a is replaced
+ * by L (the strict upper one is neither read nor written), and L^-1 goes to inv
+ * (fp64 [128, 128], lower triangular, identity past n). *info becomes 1 if a pivot
+ * is not positive (or NaN) and is left alone otherwise.
+ * Replaces: the diagonal blocks of torch.linalg.cholesky and cholesky_inverse
+ *           pare/schemes/gptq.py:203-213 */
+PMI_API int pmi_cholesky_diag(double* a, int64_t ld, int64_t n, double* inv, int32_t* info, void* stream);
+
 /* The column loop of one block, columns b0 .. b0 + count - 1 of w (fp32
  * [N, K], row-major, 16-byte aligned; w is read, not written). For each
  * column j in order: q = clamp(rint(w / s + z), 0, 15) with s, z the

@@ -50,6 +50,7 @@ SIGNATURES = {
     "pmi_gptq_group_params": (_i, [_vp, _i64, _i64, _i64, _i64, _i, _vp, _vp, _i64, _i64, _vp]),
     "pmi_gptq_block": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                             _vp]),
+    "pmi_cholesky_diag": (_i, [_vp, _i64, _i64, _vp, _vp, _vp]),
     "pmi_gptq_pack": (_i, [_vp, _vp, _vp, _i64, _i64, _vp]),
     "pmi_awq_gemm_to_storage": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     "pmi_storage_to_awq_gemm": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _i64, _i64, _i64,

@@ -1024,6 +1024,17 @@ int pmi_gptq_block(const float* w, const float* c, const int32_t* colg, const fl
                   fn);
 }
 
+int pmi_cholesky_diag(double* a, int64_t ld, int64_t n, double* inv, int32_t* info, void* stream) {
+  const char* fn = "pmi_cholesky_diag";
+  if (n < 1 || n > 128 || ld < n)
+    return fail(PMI_ERR_INVALID, "%s: need 1 <= n <= 128 and ld >= n (n=%lld ld=%lld)", fn, (long long)n,
+                (long long)ld);
+  if (!a || !inv || !info) return fail(PMI_ERR_INVALID, "%s: null buffer", fn);
+  if (!aligned(a, 8) || !aligned(inv, 8) || !aligned(info, 4))
+    return fail(PMI_ERR_INVALID, "%s: a and inv must be 8-byte aligned, info 4-byte", fn);
+  return from_hip(pmi::launch_chol_diag(a, ld, (int)n, inv, info, (hipStream_t)stream), fn);
+}
+
 int pmi_gptq_pack(const uint8_t* codes, const int32_t* inv_perm, uint8_t* packed, int64_t N,
                   int64_t K, void* stream) {
   const char* fn = "pmi_gptq_pack";

@@ -125,6 +125,9 @@ PMI_DEV void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | 0x70 | 0xF00 | ((N >> 4) << 14));
 }
 
+// s_waitcnt lgkmcnt(0), the other counters left alone (gfx9 encoding)
+PMI_DEV void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xF | 0x70 | (3 << 14)); }
+
 // s_waitcnt vmcnt(N) lgkmcnt(0): all but the N youngest vector-memory
 // operations and every LDS operation of this wave are complete
 template <int N>

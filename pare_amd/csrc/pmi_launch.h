@@ -217,6 +217,8 @@ hipError_t launch_gptq_block(const float* w, const float* c, const int32_t* colg
                              const float* scale, const float* zero, uint8_t* qt, float* et,
                              int64_t N, int64_t K, int64_t G, int64_t b0, int count,
                              hipStream_t stream);
+// Cholesky factor and its inverse of an n x n fp64 block, n <= 128.
+hipError_t launch_chol_diag(double* a, int64_t ld, int n, double* inv, int32_t* info, hipStream_t stream);
 hipError_t launch_gptq_pack(const uint8_t* qt, const int32_t* inv_perm, uint8_t* packed, int64_t N,
                             int64_t K, hipStream_t stream);
 

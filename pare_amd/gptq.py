@@ -22,9 +22,11 @@ of Frantar et al. with lazy block updates):
     code 0.
 
 Device work per layer:
-  - the Cholesky chain, in float64 through torch.linalg (rocSOLVER);
+  - the Cholesky factor of the inverse Hessian, in float64: 128-column diagonal
+    blocks in HIP (``pmi_cholesky_diag``), the rest rocBLAS GEMMs (a 4096-column
+    layer's chain through rocSOLVER took 30 of its 37.5 ms, this 5 of 8);
   - per 128-column block, the sequential column loop as one HIP launch
-    (``pmi_gptq_block``: rows on lanes, the block's C and W in LDS);
+    (``pmi_gptq_block``: a row on 16 lanes, the block's C in LDS);
   - the lazy update of the columns right of the block, as a rocBLAS GEMM;
   - a final pack (``pmi_gptq_pack``).
 The loop's rounding steps are those of gptq.py:230-249: one rounded product,
@@ -81,17 +83,80 @@ class HessianAccumulator:
         return self.H.mul(2.0 / self.n_tokens)
 
 
+def _inverse_lower(L: torch.Tensor, inv: torch.Tensor) -> torch.Tensor:
+    """Inverse of the lower triangular fp64 L [K, K] given the inverses of its
+    diagonal blocks (inv [ceil(K / BLOCK), BLOCK, BLOCK]): neighbouring blocks are
+    merged until one is left, [[A, 0], [B, C]]^-1 = [[A', 0], [-C' B A', C']],
+    all pairs of a level in one batched product each."""
+    K = L.shape[0]
+    X = torch.zeros_like(L)
+    for b, i in enumerate(range(0, K, BLOCK)):
+        n = min(BLOCK, K - i)
+        X[i:i + n, i:i + n] = inv[b, :n, :n]
+    size = BLOCK
+    while size < K:
+        pairs = K // (2 * size)                          # pairs of whole blocks
+        if pairs:
+            def blocks(M, r, c):
+                return M.as_strided((pairs, size, size), (2 * size * (K + 1), K, 1),
+                                    (r * K + c) * size)
+            low = torch.bmm(blocks(X, 1, 1), torch.bmm(blocks(L, 1, 0), blocks(X, 0, 0)))
+            blocks(X, 1, 0).copy_(low.neg_())
+        o = 2 * size * pairs
+        if K - o > size:                                 # a whole block and a shorter one
+            m = o + size
+            X[m:, o:m] = -(X[m:, m:] @ (L[m:, o:m] @ X[o:m, o:m]))
+        size *= 2
+    return X
+
+
+def _cholesky_inverse_factor(H64: torch.Tensor) -> torch.Tensor | None:
+    """Upper U with H^-1 = U^T U, fp64, or None when H is not positive definite.
+
+    With the rows and columns of H in reverse order, H' = L L^T gives H = R R^T for
+    the upper R = L in reverse order, and U = R^-1: one factorisation and one
+    triangular inverse, in place of a factorisation, an inverse of H and a
+    factorisation of that. Blocked: 128 x 128 diagonal blocks and their inverses in
+    one launch each (pmi_cholesky_diag), the panels and updates as GEMMs."""
+    lib = _lib.lib()
+    K = H64.shape[0]
+    dev = H64.device
+    A = H64.flip(0, 1).contiguous()
+    inv = torch.empty(-(-K // BLOCK), BLOCK, BLOCK, dtype=torch.float64, device=dev)
+    info = torch.zeros(1, dtype=torch.int32, device=dev)
+    stream = _stream_handle(dev)
+    with _DeviceGuard(dev):
+        for b, i in enumerate(range(0, K, BLOCK)):
+            n = min(BLOCK, K - i)
+            _lib.check(lib.pmi_cholesky_diag(A[i:, i:].data_ptr(), K, n, inv[b].data_ptr(),
+                                             info.data_ptr(), stream), "pmi_cholesky_diag")
+            if i + n < K:
+                panel = A[i + n:, i:i + n] @ inv[b, :n, :n].t()
+                A[i + n:, i:i + n] = panel
+                A[i + n:, i + n:].addmm_(panel, panel.t(), alpha=-1.0)
+    if int(info.item()):
+        return None
+    return _inverse_lower(A, inv).flip(0, 1)
+
+
 def _cholesky_chain(H: torch.Tensor, damp: float) -> torch.Tensor:
     """Upper Cholesky factor of H⁻¹ (gptq.py:203-213), float64, with the
     reference's retry at ten times the damping."""
     H64 = H.double()
-    try:
-        L = torch.linalg.cholesky(H64)
-    except torch.linalg.LinAlgError:
+    if not H64.is_cuda:
+        try:
+            L = torch.linalg.cholesky(H64)
+        except torch.linalg.LinAlgError:
+            H64.diagonal().add_(damp * 10.0)
+            L = torch.linalg.cholesky(H64)
+        return torch.linalg.cholesky(torch.cholesky_inverse(L), upper=True).float().contiguous()
+    U = _cholesky_inverse_factor(H64)
+    if U is None:
         H64.diagonal().add_(damp * 10.0)
-        L = torch.linalg.cholesky(H64)
-    Hinv = torch.cholesky_inverse(L)
-    return torch.linalg.cholesky(Hinv, upper=True).float().contiguous()
+        U = _cholesky_inverse_factor(H64)
+        if U is None:
+            raise torch.linalg.LinAlgError("the damped Hessian is not positive definite")
+    return U.float().contiguous()
 
 
 def gptq_columns(W: torch.Tensor, C: torch.Tensor, colg: torch.Tensor, scale: torch.Tensor,
@@ -163,8 +228,8 @@ def gptq_quantize(weight: torch.Tensor, hessian: torch.Tensor, group_size: int =
     H.diagonal().add_(damp)
     if act_order:                                              # gptq.py:194-200
         perm = torch.argsort(H.diagonal(), descending=True, stable=True)
-        W = W[:, perm]
-        H = H[perm][:, perm]
+        W = W.index_select(1, perm)
+        H = H[perm[:, None], perm[None, :]]
     else:
         perm = torch.arange(K, device=dev)
     W = W.contiguous()

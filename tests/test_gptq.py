@@ -425,3 +425,77 @@ def test_llama_layer_time_and_quality():
     obj_rtn = ((W - w_rtn) @ H * (W - w_rtn)).sum().item()
     print(f"objective gptq {obj:.4g} rtn {obj_rtn:.4g}", flush=True)
     assert obj < 0.8 * obj_rtn
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [16, 112, 128, 144, 256, 384, 400, 640, 1408])
+def test_device_factor_of_the_inverse(K):
+    """The blocked factor of H^-1 (one block, whole blocks, a short last block, an
+    odd number of blocks) against the chain through torch.linalg in float64 on
+    the CPU. Both are backward stable: they differ by a few K 2^-53 cond(H),
+    here below K 2^-53 1e4, and the fp32 results by one rounding."""
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(2 * K, K, generator=g, dtype=torch.float64)
+    x = (x + 0.5 * x.roll(1, dims=1)) * torch.exp(0.5 * torch.randn(K, generator=g, dtype=torch.float64))
+    H = x.t() @ x / K
+    H.diagonal().add_(0.01 * H.diagonal().mean())
+    U = G._cholesky_inverse_factor(H.to("cuda"))
+    want = torch.linalg.cholesky(torch.cholesky_inverse(torch.linalg.cholesky(H)), upper=True)
+    assert float((U.cpu() - want).norm() / want.norm()) < K * 2.0 ** -53 * 1e4
+    assert not torch.any(torch.tril(U, -1))
+    C = G._cholesky_chain(H.float().to("cuda"), 0.0).cpu()
+    assert C.dtype == torch.float32 and C.is_contiguous()
+
+
+@pytest.mark.gpu
+def test_device_factor_retries_and_fails_like_the_library():
+    """Not positive definite: a retry with ten times the damping on the
+    diagonal, then LinAlgError."""
+    K = 272
+    H = torch.eye(K, device="cuda")
+    H[200, 200] = -0.5
+    C = G._cholesky_chain(H, 0.1)             # -0.5 + 1 on the diagonal
+    want = torch.full((K,), 2.0).rsqrt()
+    want[200] = 0.5 ** -0.5
+    assert torch.allclose(C.cpu(), torch.diag(want))
+    with pytest.raises(torch.linalg.LinAlgError):
+        G._cholesky_chain(H, 0.01)
+    H[200, 200] = float("nan")
+    with pytest.raises(torch.linalg.LinAlgError):
+        G._cholesky_chain(H, 0.1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,b0,count", [(1, 16, 0, 16), (15, 128, 0, 128), (17, 144, 128, 16),
+                                          (33, 240, 128, 112), (300, 256, 128, 128)])
+def test_block_kernel_bit_exact_edges(N, K, b0, count):
+    """One block on its own (short blocks, rows that do not fill a workgroup,
+    groups in any order per column) equals the oracle's column loop bit for
+    bit: codes and errors."""
+    gs = 16
+    rng = np.random.default_rng(N + K)
+    W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    C = np.triu(rng.standard_normal((K, K)) * 0.05).astype(np.float32)
+    C[np.arange(K), np.arange(K)] = rng.uniform(0.3, 3.0, K).astype(np.float32)
+    colg = rng.permutation(K).astype(np.int32) // gs
+    scale = rng.uniform(1e-3, 6e-3, (N, K // gs)).astype(np.float32)
+    zero = rng.integers(0, 16, (N, K // gs)).astype(np.float32)
+    E = np.zeros((count, N), np.float32)
+    Wb = W[:, b0:b0 + count].copy()
+    Q = np.zeros((count, N), np.uint8)
+    for k in range(count):
+        s, z = scale[:, colg[b0 + k]], zero[:, colg[b0 + k]]
+        q = np.clip(np.rint(Wb[:, k] / s + z), np.float32(0), np.float32(15))
+        e = (Wb[:, k] - (q - z) * s) / C[b0 + k, b0 + k]
+        Q[k], E[k] = q, e
+        Wb[:, k + 1:] -= e[:, None] * C[b0 + k, b0 + k + 1:b0 + count][None, :]
+    d = [torch.from_numpy(a).to("cuda") for a in (W, C, colg, scale, zero)]
+    codes = torch.zeros(K, N, dtype=torch.uint8, device="cuda")
+    err = torch.zeros(count, N, device="cuda")
+    rc = _lib.lib().pmi_gptq_block(*(t.data_ptr() for t in d), codes.data_ptr(), err.data_ptr(), N, K,
+                                   K // gs, b0, count, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(codes[b0:b0 + count].cpu().numpy(), Q)
+    assert not codes[:b0].any() and not codes[b0 + count:].any()
+    assert np.array_equal(err.cpu().numpy().view(np.uint32), E.view(np.uint32))
