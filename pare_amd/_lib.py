@@ -129,6 +129,25 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The host extension (csrc/host_ext.cpp), bound to the library's entry
+    points; raises RuntimeError if it has not been built."""
+    global _host
+    if _host is None:
+        handle = lib()
+        try:
+            from . import _host as ext
+        except ImportError as e:
+            raise RuntimeError("pare_amd/_host is not built; run `python -m pare_amd.build`") from e
+        ext.bind(*(ctypes.cast(getattr(handle, fn), ctypes.c_void_p).value for fn in (
+            "pmi_matmul_w4a16", "pmi_matmul_kernel_choice", "pmi_matmul_best_workspace_bytes")))
+        _host = ext
+    return _host
+
+
 def last_error() -> str:
     return lib().pmi_last_error().decode("utf-8", "replace")
 

@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -24,6 +25,10 @@ LIB_PATH = PKG_DIR / LIB_NAME
 SOURCES = ["capi.hip", "w4a16_gemv.hip", "w4a16_gemm.hip", "w4a16_gemm64.hip", "w4a16_skinny.hip",
            "w4a16_layout.hip", "decode_ops.hip", "gptq.hip", "probes.hip",
            "w4a16_tgemm.hip", "w4a16_bgemm.hip"]
+
+# The host path of a matmul call, a CPython extension against torch's headers.
+HOST_SOURCE = "host_ext.cpp"
+HOST_PATH = PKG_DIR / f"_host{sysconfig.get_config_var('EXT_SUFFIX')}"
 
 HIPCC_FLAGS = [
     "-O3",
@@ -62,8 +67,22 @@ def _run(cmd: list[str], verbose: bool) -> str:
     return res.stderr
 
 
+def _host_command() -> list[str]:
+    from torch.utils import cpp_extension as ext
+    import torch
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "g++"
+    inc = [f"-I{d}" for d in [*ext.include_paths(), sysconfig.get_paths()["include"]]]
+    libs = [f"-L{d}" for d in ext.library_paths()]
+    return [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            "-DTORCH_API_INCLUDE_EXTENSION_H", *inc, str(CSRC / HOST_SOURCE), *libs,
+            "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python", "-o", f"{HOST_PATH}.tmp"]
+
+
 def build(verbose: bool = False, extra_flags: list[str] | None = None) -> Path:
-    """Compiles every HIP source into ``pare_amd/libpare_amd.so`` (always rebuilds).
+    """Compiles every HIP source into ``pare_amd/libpare_amd.so`` and the host
+    extension ``pare_amd/_host*.so`` (always rebuilds).
 
     Each source is compiled to an object of its own in parallel (``_build/``
     at the repository root, ignored by git), then the objects are linked."""
@@ -76,9 +95,12 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None) -> Path:
     for src in SOURCES:
         obj = obj_dir / (Path(src).stem + ".o")
         jobs.append((obj, [hipcc, *flags, inc, "-c", str(CSRC / src), "-o", str(obj)]))
-    workers = max(1, min(len(jobs), int(os.environ.get("MAX_JOBS", "0") or 0) or os.cpu_count() or 1))
+    workers = max(1, min(len(jobs) + 1, int(os.environ.get("MAX_JOBS", "0") or 0) or os.cpu_count() or 1))
     with ThreadPoolExecutor(max_workers=workers) as pool:
+        host = pool.submit(_run, _host_command(), verbose)
         logs = list(pool.map(lambda j: _run(j[1], verbose), jobs))
+        logs.append(host.result())
+    os.replace(f"{HOST_PATH}.tmp", HOST_PATH)
     tmp = LIB_PATH.with_suffix(".so.tmp")
     logs.append(_run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC",
                       *[str(o) for o, _ in jobs], "-o", str(tmp)], verbose))

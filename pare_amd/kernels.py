@@ -114,6 +114,18 @@ def _workspace(dev: torch.device, stream: int, nbytes: int) -> torch.Tensor | No
     return ws
 
 
+def host_matmul(x, w, scales, zeros, group_size, perm, perm16, sz_gm, w_tiled, *,
+                build_tiled=False, cast=False, bf16=False, bias=None):
+    """A plain matmul call through the host extension (csrc/host_ext.cpp), or
+    None where it is not one: the caller's general path then takes it."""
+    dev = torch._C._cuda_getDevice()
+    stream = torch._C._cuda_getCurrentRawStream(dev)
+    s_gm, z_gm = (None, None) if sz_gm is None else sz_gm
+    return _lib.host().matmul(x, w, scales, zeros, group_size, perm, perm16, s_gm, z_gm, w_tiled,
+                              build_tiled, cast, bf16, bias, dev, stream,
+                              lambda nbytes: _workspace(x.device, stream, nbytes))
+
+
 def matmul_w4a16(
     x: torch.Tensor,
     packed_weight: torch.Tensor,
@@ -151,6 +163,11 @@ def matmul_w4a16(
         raise RuntimeError("matmul_w4a16 requires HIP (cuda) tensors.")
     assert x.is_contiguous(), "x must be contiguous"
     assert x.dtype == torch.float16, f"x must be float16, got {x.dtype}"
+    if out is None and x.dim() == 2 and (sz_gm is None or len(sz_gm) == 2):
+        y = host_matmul(x, packed_weight, scales, zeros, group_size, perm, perm16, sz_gm, w_tiled,
+                        bf16=False)
+        if y is not None:
+            return y
     return _matmul(x, packed_weight, scales, zeros, group_size, perm, perm16, sz_gm, w_tiled, out)
 
 
@@ -180,6 +197,11 @@ def matmul_w4a16_bf16(
         raise RuntimeError("matmul_w4a16_bf16 requires HIP (cuda) tensors.")
     assert x.is_contiguous(), "x must be contiguous"
     assert x.dtype == torch.bfloat16, f"x must be bfloat16, got {x.dtype}"
+    if out is None and x.dim() == 2 and (sz_gm is None or len(sz_gm) == 2):
+        y = host_matmul(x, packed_weight, scales, zeros, group_size, perm, perm16, sz_gm, w_tiled,
+                        bf16=True)
+        if y is not None:
+            return y
     return _matmul(x, packed_weight, scales, zeros, group_size, perm, perm16, sz_gm, w_tiled, out)
 
 

@@ -21,7 +21,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .config import QuantConfig, is_int4, kernel_group_size
-from .kernels import kernel_choice, matmul_w4a16, matmul_w4a16_bf16
+from .kernels import host_matmul, kernel_choice, matmul_w4a16, matmul_w4a16_bf16
 from .pack import (dequantize_int4, perm_from_g_idx, perm_u16, repack_int4_for_kernel,
                    sz_group_major, tile_w4a16, tiled_supported, zeros_to_u8)
 
@@ -109,7 +109,8 @@ class QuantizedLinear(nn.Module):
             raise RuntimeError("pare_amd.QuantizedLinear runs on the HIP device only "
                                "(no CPU fallback); move the module and input to cuda")
         if getattr(self, "use_kernel", False):
-            return self._forward_kernel(x)
+            y = self._forward_host(x)
+            return self._forward_kernel(x) if y is None else y
         weight = self.dequantize(dtype=x.dtype)
         return F.linear(x, weight, self.bias)
 
@@ -129,7 +130,8 @@ class QuantizedLinear(nn.Module):
         # the 16-bit copy the GEMV's act_order gather reads (None past K = 65536)
         self._perm16 = perm_u16(perm) if perm is not None else None
         zero_u8 = zeros_to_u8(self.zero)
-        self._kernel_cache = (self._stamp(), zero_u8, perm, sz_group_major(self.scale, zero_u8))
+        self._kernel_cache = (self._stamp(), zero_u8, perm, sz_group_major(self.scale, zero_u8),
+                              tiled_supported(self.out_features, self.in_features, gs))
 
     def _kernel_buffers(self):
         """Kernel-layout weight, u8 zeros, group-major scales/zeros and the
@@ -168,6 +170,26 @@ class QuantizedLinear(nn.Module):
             raise ValueError("kernel-layout weight must be uint8 with the packed weight's shape "
                              "and device")
         self._build_kernel_cache(w_kernel.contiguous())
+
+    def _forward_host(self, x: torch.Tensor) -> torch.Tensor | None:
+        """The kernel forward of a layer whose copies exist, through the host
+        extension; None where anything has to be built, converted or refused
+        (``_forward_kernel`` then does it). The buffers are read from the module's
+        dict: as attributes they go through ``nn.Module.__getattr__``."""
+        d = self.__dict__
+        cache = d.get("_kernel_cache")
+        if cache is None:
+            return None
+        b = self._buffers
+        packed, scale, zero = b["packed_weight"], b["scale"], b["zero"]
+        if cache[0] != (packed.device, packed.data_ptr(), packed._version, zero._version,
+                        scale._version):
+            return None
+        params = self._parameters
+        return host_matmul(x, d["_packed_weight_kernel"], scale, cache[1], self._group_size(), cache[2],
+                           d["_perm16"], cache[3], d["_packed_weight_tiled"], build_tiled=cache[4],
+                           cast=True, bf16=d.get("native_bf16", False),
+                           bias=params["bias"] if "bias" in params else d.get("bias"))
 
     def _forward_kernel(self, x: torch.Tensor) -> torch.Tensor:
         """pare/layers/linear.py:140-159 with the HIP kernels. bf16 inputs are

@@ -1,0 +1,117 @@
+"""The host extension's matmul call against the general Python path: the same
+bits, dtypes and shapes where it takes a call, the same errors where it does
+not."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import pare_amd as P
+from pare_amd import kernels as KN
+from pare_amd.config import QuantConfig
+from pare_amd.linear import QuantizedLinear
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+
+
+def _layer(N, K, gs, bias=None, act_order=False, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    w = torch.randn(N, K, generator=g, device=DEV) * 0.02
+    packed, s, z = P.rtn_quantize(w, gs)
+    g_idx = None
+    if act_order:
+        g_idx = (torch.randperm(K, generator=g, device=DEV) // gs).to(torch.int32)
+    return QuantizedLinear(packed, s, z, QuantConfig(bits=4, scheme="rtn", group_size=gs), bias, K, N,
+                           use_kernel=True, g_idx=g_idx)
+
+
+@pytest.mark.parametrize("shape", [(1,), (1, 1), (2, 3), (4, 1, 5), (70,), ()])
+@pytest.mark.parametrize("dtype,native", [(torch.float16, False), (torch.bfloat16, False),
+                                          (torch.bfloat16, True), (torch.float32, False)])
+@pytest.mark.parametrize("N,K,gs,act_order", [(512, 1536, 128, False), (1028, 2048, 64, False),
+                                              (260, 384, 128, True), (66, 256, 32, False)])
+def test_module_forward_equals_the_general_path(N, K, gs, act_order, dtype, native, shape):
+    for bias in (None, torch.randn(N, device=DEV).to(dtype)):
+        layer = _layer(N, K, gs, bias, act_order)
+        layer.native_bf16 = native
+        x = torch.randn(*shape, K, device=DEV).to(dtype)
+        with torch.no_grad():
+            first = layer(x)                          # builds the copies: general path
+            fast = layer._forward_host(x)
+            want = layer._forward_kernel(x)
+        assert fast is not None
+        for y in (first, fast):
+            assert y.dtype == want.dtype and y.shape == want.shape and y.is_contiguous()
+            assert torch.equal(y, want)
+
+
+def test_module_inputs_the_host_path_converts_or_leaves():
+    layer = _layer(512, 1536, 128)
+    x = torch.randn(6, 1536, device=DEV).half()
+    want = layer(x)
+    strided = torch.empty(6, 3072, device=DEV).half()[:, ::2].copy_(x)
+    odd = torch.empty(6 * 1536 + 1, device=DEV).half()[1:].view(6, 1536).copy_(x)
+    turned = x.t().contiguous().t()
+    for v in (strided, odd, turned):
+        assert torch.equal(layer._forward_host(v), want)
+        assert torch.equal(layer(v), want)
+    # left to the general path: empty inputs, other dtypes, changed weights
+    assert layer._forward_host(x[:0]) is None and layer(x[:0]).shape == (0, 512)
+    assert layer._forward_host(x.double()) is None and layer(x.double()).dtype == torch.float64
+    layer.scale.mul_(2.0)
+    assert layer._forward_host(x) is None
+    assert torch.allclose(layer(x), 2 * want, rtol=2e-3, atol=1e-3)
+    assert layer._forward_host(x) is not None
+    with pytest.raises(RuntimeError, match="HIP device"):
+        layer(x.cpu())
+    with pytest.raises(RuntimeError):
+        layer(torch.randn(2, 1000, device=DEV).half())
+
+
+def test_bias_keeps_its_gradient_and_dtype():
+    layer = _layer(256, 1536, 128, torch.randn(256, device=DEV))
+    x = torch.randn(3, 1536, device=DEV).half()
+    layer(x)
+    y = layer(x)                                     # fp16 result + fp32 bias
+    assert y.dtype == torch.float32 and y.requires_grad
+    y.sum().backward()
+    assert torch.equal(layer.bias.grad, torch.full((256,), 3.0, device=DEV))
+
+
+def test_operator_errors_are_the_general_paths():
+    layer = _layer(256, 1536, 128)
+    w, z, _, sz = layer._kernel_buffers()
+    s = layer.scale
+    x = torch.randn(4, 1536, device=DEV).half()
+    want = P.matmul_w4a16(x, w, s, z, 128)
+    assert torch.equal(KN._matmul(x, w, s, z, 128, None, None, None, None, None), want)
+    assert torch.equal(P.matmul_w4a16(x, w, s, z.float(), 128), want)   # fp32 zeros: general path
+    out = torch.empty(4, 256, device=DEV, dtype=torch.float16)
+    assert P.matmul_w4a16(x, w, s, z, 128, out=out) is out and torch.equal(out, want)
+    bad = [dict(x=x[0]), dict(x=x.t()), dict(x=x.float()), dict(w=w[:, :-1]), dict(w=w.to(torch.int8)),
+           dict(s=s[:-1]), dict(s=s.reshape(256, 1, 12)), dict(gs=100), dict(sz_gm=(sz[0].t(), sz[1].t())),
+           dict(perm16=torch.zeros(1536, dtype=torch.int16, device=DEV)),
+           dict(w_tiled=torch.zeros(16, dtype=torch.uint8, device=DEV)),
+           dict(perm=torch.zeros(1536, dtype=torch.int64, device=DEV))]
+    for kw in bad:
+        args = {"x": x, "w": w, "s": s, "gs": 128, **kw}
+        extra = {k: v for k, v in kw.items() if k not in ("x", "w", "s", "gs")}
+        with pytest.raises((AssertionError, RuntimeError, IndexError)):
+            P.matmul_w4a16(args["x"], args["w"], args["s"], z, args["gs"], **extra)
+
+
+def test_vmap_and_subclasses_are_not_read_as_plain_tensors():
+    layer = _layer(256, 1536, 128)
+    x = torch.randn(4, 1536, device=DEV).half()
+    want = layer(x)
+
+    class Sub(torch.Tensor):
+        pass
+
+    sub = x.as_subclass(Sub)
+    assert torch.equal(torch.as_tensor(layer(sub)).as_subclass(torch.Tensor), want)
+    with pytest.raises(RuntimeError):
+        torch.vmap(layer)(x)
