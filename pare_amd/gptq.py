@@ -121,7 +121,10 @@ def _cholesky_inverse_factor(H64: torch.Tensor) -> torch.Tensor | None:
     lib = _lib.lib()
     K = H64.shape[0]
     dev = H64.device
-    A = H64.flip(0, 1).contiguous()
+    # transposed as well: the lower triangle of H is the one that is read, as
+    # torch.linalg reads it (a Gram matrix from a GEMM is symmetric only to its
+    # rounding)
+    A = H64.t().flip(0, 1).contiguous()
     inv = torch.empty(-(-K // BLOCK), BLOCK, BLOCK, dtype=torch.float64, device=dev)
     info = torch.zeros(1, dtype=torch.int32, device=dev)
     stream = _stream_handle(dev)

@@ -439,6 +439,8 @@ def test_device_factor_of_the_inverse(K):
     x = (x + 0.5 * x.roll(1, dims=1)) * torch.exp(0.5 * torch.randn(K, generator=g, dtype=torch.float64))
     H = x.t() @ x / K
     H.diagonal().add_(0.01 * H.diagonal().mean())
+    # only the lower triangle counts, as for torch.linalg
+    H = H + torch.triu(torch.randn(K, K, generator=g, dtype=torch.float64), 1) * 1e-3
     U = G._cholesky_inverse_factor(H.to("cuda"))
     want = torch.linalg.cholesky(torch.cholesky_inverse(torch.linalg.cholesky(H)), upper=True)
     assert float((U.cpu() - want).norm() / want.norm()) < K * 2.0 ** -53 * 1e4
