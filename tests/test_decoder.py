@@ -640,3 +640,24 @@ def test_shared_workspaces_alternate_large_and_small_shapes():
         argmax_into(x, out)
         assert torch.equal(out, x.argmax(-1)), ("argmax", rows)
         print(f"[workspace] B={B} argmax rows={rows} ok", flush=True)
+
+
+@pytest.mark.parametrize("B,T,H,KV,L", [(1, 1, 4, 1, 3), (2, 5, 8, 2, 7), (3, 33, 16, 16, 40)])
+def test_rope_kv_wide_equals_the_pairwise_kernel(B, T, H, KV, L):
+    """Eight pairs per thread (16-byte aligned buffers) against the kernel that
+    takes a pair per thread, which runs when qkv starts at an odd element: the
+    same bits in q and in both caches, positions in any order."""
+    D = 128
+    g = torch.Generator(device=DEV).manual_seed(B * T)
+    qkv = torch.randn(B * T, (H + 2 * KV) * D, generator=g, device=DEV).half()
+    odd = torch.empty(qkv.numel() + 1, dtype=torch.float16, device=DEV)[1:].view(qkv.shape).copy_(qkv)
+    cos, sin = rope_tables(D, 500000.0, L, DEV)
+    pos = torch.randperm(L, generator=g, device=DEV)[:T]
+    got = []
+    for src in (qkv, odd):
+        ck = torch.zeros(B, KV, L, D, dtype=torch.float16, device=DEV)
+        cv = torch.zeros_like(ck)
+        got.append((rope_kv(src, cos, sin, pos, ck, cv, B, T, H, KV, D), ck, cv))
+    for a, b in zip(*got):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    assert got[0][1].abs().sum() > 0
