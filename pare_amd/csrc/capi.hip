@@ -215,11 +215,15 @@ int pmi_matmul_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t group_size
     if (c.splits > 1 && c.ntw == 4) return 5;
   }
   // Many activation rows (prefill): the big-tile GEMM, 256 weight rows x 128
-  // activation rows per workgroup, where its tiles fill three quarters of
-  // the CUs in one pass or more.
+  // activation rows per workgroup, where its tiles fill three quarters of the
+  // CUs, or, with K split over fewer tiles, from M N K = 1.8e10 on (us, register-
+  // streamed GEMM against it): 4096 x 14336 at M = 256 / 384 / 640 / 1024 39.4 / 56.7
+  // / 109 / 133 against 43.4 / 54.2 / 80 / 112; 4096 x 4096 at M = 1024 / 1152 43.1 / 59.3
+  // against 45.0 / 56.2; 1024 x 14336 at M = 1024 / 1536 38.6 / 63.4 against 41.3 /
+  // 53.8; 7096 x 5504 at M = 512 / 640 50.7 / 73.4 against 51.5 / 74.6.
   if (has_tiled && M > 64 && group_size % 128 == 0 && pmi::tgemm_supported(M, N, K, group_size)) {
     const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, group_size);
-    if (b.ok && (int64_t)b.n_bands * b.grid_m * 4 >= 3 * cus) return 6;
+    if (b.ok && ((int64_t)b.n_bands * b.grid_m * 4 >= 3 * cus || M * N * K >= 18000000000ll)) return 6;
   }
   // Past 64 rows on narrow layers, while the tiled GEMM's 64-row blocks still
   // take one pass over the CUs: against the register-streamed GEMM, whose K
@@ -739,6 +743,14 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
   if ((choice == 5 || choice == 6) && !aligned(y, 8)) {
     if (forced) return fail(PMI_ERR_INVALID, "%s: the tiled GEMM needs y 8-byte aligned", fn);
     choice = pmi_matmul_kernel_choice(M, N, K, group_size, perm ? PMI_CHOICE_PERM : 0);
+  }
+  // without the workspace of its K split the big-tile GEMM leaves such a call
+  // to the kernel it would run on without the tiled copy
+  if (choice == 6 && !forced) {
+    const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, group_size);
+    const size_t room = pmi::kWsCounterBytes + (perm ? pmi::ws_perm_bytes(M, K) : 0) + b.ws_split;
+    if ((int64_t)b.n_bands * b.grid_m * 4 < 3 * pmi::device_cu_count() && workspace_bytes < room)
+      choice = pmi_matmul_kernel_choice(M, N, K, group_size, perm ? PMI_CHOICE_PERM : 0);
   }
   if (choice == 6) {
     if (!has_tiled || !pmi::tgemm_supported(M, N, K, group_size) || group_size % 128 != 0 ||

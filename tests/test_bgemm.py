@@ -65,6 +65,8 @@ def _bound(x, w_hat, s, gs, bf16):
     (25, 260, 384, 128, False, False, False), (60, 1028, 1408, 128, False, False, True),
     (33, 64, 128, 64, False, False, False), (225, 516, 1152, 64, False, False, False),
     (97, 900, 160 * 4, 32, False, False, False), (12, 16644, 2048, 32, False, False, True),
+    # fp16 with the copies: K split over few tiles, from M N K = 1.8e10
+    (643, 2060, 14336, 128, False, True, False), (1153, 4096, 4096, 128, False, True, True),
     # fp16 without the copies, large enough to leave the register-streamed GEMM
     (769, 5636, 4096, 128, False, False, False),
 ])
@@ -126,6 +128,33 @@ def test_bgemm_route_needs_no_workspace_and_no_alignment_of_y():
         assert call(y, w) == 0, _lib.last_error()
         torch.cuda.synchronize()
         assert torch.equal(y.view(M, N).view(torch.int16), want.view(torch.int16))
+
+
+def test_bgemm_split_without_its_workspace_runs_elsewhere():
+    """Few tiles and no room for their split: the call runs on the kernel that
+    it would run on without the tiled copy (same bits), through the C ABI."""
+    M, N, K, gs = 643, 2060, 14336, 128
+    L = _lib.lib()
+    assert L.pmi_matmul_kernel_choice(M, N, K, gs, _lib.PMI_CHOICE_TILED) == 6
+    assert L.pmi_matmul_kernel_choice(M, N, K, gs, 0) == 4
+    g = torch.Generator(device=DEV).manual_seed(4)
+    wk = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8, device=DEV)
+    s = torch.rand(N, K // gs, generator=g, device=DEV) * 0.01 + 1e-3
+    z = torch.randint(0, 16, (N, K // gs), generator=g, dtype=torch.uint8, device=DEV)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    s_gm, z_gm = P.sz_group_major(s, z)
+    wt = P.tile_w4a16(wk, gs)
+    stream = torch.cuda.current_stream().cuda_stream
+    out = []
+    for tiled in (wt.data_ptr(), None):
+        y = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+        rc = L.pmi_matmul_w4a16(x.data_ptr(), _lib.PMI_F16, wk.data_ptr(), s.data_ptr(), z.data_ptr(),
+                                _lib.PMI_U8, None, None, s_gm.data_ptr(), z_gm.data_ptr(), tiled,
+                                y.data_ptr(), _lib.PMI_F16, M, N, K, gs, None, 0, stream)
+        assert rc == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        out.append(y)
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
 @pytest.mark.parametrize("bf16,gs", [(True, 128), (False, 64)])
