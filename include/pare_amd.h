@@ -260,6 +260,16 @@ PMI_API int pmi_matmul_w4a16_gate_up_silu(const void* x, const uint8_t* w_tiled,
 /* 1 when pmi_matmul_w4a16_gate_up_silu runs this shape, else 0. Host-only. */
 PMI_API int pmi_gate_up_silu_supported(int64_t M, int64_t N, int64_t K, int64_t group_size);
 
+/* The same product for many activation rows (prefill), on the big-tile GEMM:
+ * for the shapes pmi_gate_up_silu_rows_supported accepts (more than 64 rows, N %
+ * 64 == 0, group_size % 128 == 0, enough tiles to fill the CUs), else
+ * PMI_ERR_UNSUPPORTED. y equals pmi_matmul_w4a16 followed by pmi_silu_mul_f16 bit
+ * for bit. No reference counterpart. */
+PMI_API int pmi_matmul_w4a16_gate_up_silu_rows(const void* x, const uint8_t* w_tiled, const float* scales_gm,
+                                               const uint8_t* zeros_gm, void* y, int64_t M, int64_t N,
+                                               int64_t K, int64_t group_size, void* stream);
+PMI_API int pmi_gate_up_silu_rows_supported(int64_t M, int64_t N, int64_t K, int64_t group_size);
+
 /* y = (RMSNorm(x + residual) * norm_weight) . dequant(W)^T for M <= 4: a
  * decoder's residual add and pre-norm fused into the GEMV that consumes them.
  * x, residual (nullable), h_out: fp16 [M, K]; norm_weight fp16 [K]. With a

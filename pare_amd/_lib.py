@@ -69,6 +69,8 @@ SIGNATURES = {
     "pmi_tgemm_splits": (_i, [_i64, _i64, _i64, _i64, _i]),
     "pmi_matmul_w4a16_gate_up_silu": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "pmi_gate_up_silu_supported": (_i, [_i64, _i64, _i64, _i64]),
+    "pmi_gate_up_silu_rows_supported": (_i, [_i64, _i64, _i64, _i64]),
+    "pmi_matmul_w4a16_gate_up_silu_rows": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "pmi_matmul_w4a16_tiled_rmsnorm": (_i, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp,
                                             _i64, _i64, _i64, _i64, _i, _vp]),
     "pmi_tiled_rmsnorm_supported": (_i, [_i64, _i64, _i64, _i64, _i]),

@@ -310,6 +310,30 @@ int pmi_matmul_w4a16_gate_up_silu(const void* x, const uint8_t* w_tiled, const f
                   fn);
 }
 
+int pmi_gate_up_silu_rows_supported(int64_t M, int64_t N, int64_t K, int64_t group_size) {
+  if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || K % group_size != 0) return 0;
+  return pmi::tgemm_supported(M, N, K, group_size) && pmi::bgemm_glu_supported(M, N, K, group_size) ? 1 : 0;
+}
+
+int pmi_matmul_w4a16_gate_up_silu_rows(const void* x, const uint8_t* w_tiled, const float* scales_gm,
+                                       const uint8_t* zeros_gm, void* y, int64_t M, int64_t N,
+                                       int64_t K, int64_t group_size, void* stream) {
+  const char* fn = "pmi_matmul_w4a16_gate_up_silu_rows";
+  if (int rc = check_shape(N, K, group_size, fn)) return rc;
+  if (M < 0) return fail(PMI_ERR_INVALID, "%s: M < 0", fn);
+  if (M == 0 || N == 0) return ok();
+  if (!pmi_gate_up_silu_rows_supported(M, N, K, group_size))
+    return fail(PMI_ERR_UNSUPPORTED, "%s: shape not on the unsplit big-tile GEMM (M=%lld N=%lld K=%lld gs=%lld; "
+                "see pmi_gate_up_silu_rows_supported)", fn, (long long)M, (long long)N, (long long)K,
+                (long long)group_size);
+  if (!x || !w_tiled || !scales_gm || !zeros_gm || !y) return fail(PMI_ERR_INVALID, "%s: null buffer", fn);
+  if (!aligned(x, 16) || !aligned(w_tiled, 16) || !aligned(scales_gm, 16) || !aligned(zeros_gm, 4) || !aligned(y, 4))
+    return fail(PMI_ERR_INVALID, "%s: x, w_tiled and scales_gm must be 16-byte aligned, zeros_gm and y 4-byte", fn);
+  return from_hip(pmi::launch_bgemm(x, w_tiled, nullptr, scales_gm, zeros_gm, y, M, N, K, group_size, false,
+                                    nullptr, 0, 0, (hipStream_t)stream, true),
+                  fn);
+}
+
 int pmi_tiled_rmsnorm_supported(int64_t M, int64_t N, int64_t K, int64_t group_size, int glu) {
   if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || K % group_size != 0) return 0;
   return pmi::tgemm_norm_supported(M, N, K, group_size, glu != 0) ? 1 : 0;

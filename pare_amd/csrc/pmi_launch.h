@@ -266,7 +266,11 @@ BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16 
 // workspace: the row sums (bf16) and partial tiles, from ws_offset on.
 hipError_t launch_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w_kernel, const float* scales_gm,
                         const uint8_t* zeros_gm, void* y, int64_t M, int64_t N, int64_t K, int64_t gs,
-                        bool bf16, void* workspace, size_t ws_bytes, size_t ws_offset, hipStream_t stream);
+                        bool bf16, void* workspace, size_t ws_bytes, size_t ws_offset, hipStream_t stream,
+                        bool glu = false);
+// y [M, N / 2] = silu(gate) * up from a tiled gate/up weight in the row order of
+// tgemm_glu (launch_bgemm with glu), where the tiles fill the CUs unsplit.
+bool bgemm_glu_supported(int64_t M, int64_t N, int64_t K, int64_t gs);
 // perm: act_order columns, gathered in the kernel (tgemm_gather_supported), or null;
 // perm16 (nullable, with perm): its 16-bit copy, which the gather then reads instead.
 // workspace: counters (zero between calls) at its start and the split-K partial

@@ -74,6 +74,7 @@ struct BgemmArgs {
   int n_panels, n_bands, grid_m, splits;
   int chunk;             // workgroups per XCD
   int sums_ld;
+  int glu;               // fp16, tiled, 128-column groups: y [M, N / 2] = silu(gate) * up
 };
 
 template <int MT, int KSG, bool BF>
@@ -153,6 +154,20 @@ PMI_DEV void store_rows(uint16_t* __restrict__ y, const f32x4* v, int m, int M, 
       o[q] = v0 | (v1 << 16);
     }
     *reinterpret_cast<u32x2*>(y + (size_t)(m + e) * N + row0) = o;
+  }
+}
+
+// The same rows of a gate/up weight in pmi_matmul_w4a16_gate_up_silu's row order
+// (v[0], v[1] gate, v[2], v[3] up of output columns col, col + 1): silu(gate) * up
+// with the roundings of the plain matmul followed by pmi_silu_mul_f16.
+PMI_DEV void store_rows_glu(uint16_t* __restrict__ y, const f32x4* v, int m, int M, int ld, int col) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (m + e >= M) continue;
+    uint32_t h[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h[j] = __builtin_bit_cast(uint16_t, f32_to_f16_rne(v[j][e]));
+    *reinterpret_cast<uint32_t*>(y + (size_t)(m + e) * ld + col) = glu_pair(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
   }
 }
 
@@ -516,7 +531,14 @@ __global__ __launch_bounds__(256 * KG, 2) void w4a16_bgemm_kernel(BgemmArgs a) {
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     if (KG == 2 && (i < H) != (kgrp == 0)) continue;
-    store_rows<BF>(a.y, acc[i], m0 + 16 * i + 4 * (l >> 4), M, N, row0);
+    const int m = m0 + 16 * i + 4 * (l >> 4);
+    if constexpr (!BF && !RM && KSG == 4) {
+      if (a.glu) {
+        store_rows_glu(a.y, acc[i], m, M, N / 2, 32 * p + 2 * (l & 15));
+        continue;
+      }
+    }
+    store_rows<BF>(a.y, acc[i], m, M, N, row0);
   }
 }
 
@@ -640,12 +662,20 @@ BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16)
   return c;
 }
 
+bool bgemm_glu_supported(int64_t M, int64_t N, int64_t K, int64_t gs) {
+  if (M <= 64 || N % 64 != 0 || gs % 128 != 0) return false;
+  const BgemmConfig c = bgemm_config(M, N, K, gs);
+  return c.ok && c.splits == 1 && (int64_t)c.n_bands * c.grid_m * 4 >= 3 * (int64_t)device_cu_count();
+}
+
 hipError_t launch_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w_kernel, const float* scales_gm,
                         const uint8_t* zeros_gm, void* y, int64_t M, int64_t N, int64_t K, int64_t gs,
-                        bool bf16, void* workspace, size_t ws_bytes, size_t ws_offset, hipStream_t stream) {
+                        bool bf16, void* workspace, size_t ws_bytes, size_t ws_offset, hipStream_t stream,
+                        bool glu) {
   BgemmConfig c = bgemm_config(M, N, K, gs, bf16);
-  if (!c.ok) return hipErrorInvalidValue;
+  if (!c.ok || (glu && !bgemm_glu_supported(M, N, K, gs))) return hipErrorInvalidValue;
   BgemmArgs a{};
+  a.glu = glu;
   size_t off = ws_offset;
   if (bf16) {
     if (!workspace || ws_bytes < off + c.ws_sums) return hipErrorInvalidValue;

@@ -36,8 +36,9 @@ import torch.nn.functional as F
 
 from . import _lib
 from .config import QuantConfig
-from .kernels import (_stream_handle, gate_up_silu_supported, glu_row_order, kernel_choice,
-                      matmul_w4a16_gate_up_silu, matmul_w4a16_glu, matmul_w4a16_prenormed,
+from .kernels import (_stream_handle, gate_up_silu_rows_supported, gate_up_silu_supported,
+                      glu_row_order, kernel_choice, matmul_w4a16_gate_up_silu,
+                      matmul_w4a16_gate_up_silu_rows, matmul_w4a16_glu, matmul_w4a16_prenormed,
                       matmul_w4a16_residual, matmul_w4a16_rmsnorm, matmul_w4a16_tiled_rmsnorm,
                       residual_stats_count, tiled_rmsnorm_supported)
 from .pack import sz_group_major, tile_w4a16
@@ -437,7 +438,21 @@ class DecoderLayer(nn.Module):
             act = matmul_w4a16_gate_up_silu(n2.reshape(M, -1).contiguous(), w_t, sz,
                                             gu._group_size(), gu.out_features)
             return self.down(act.reshape(B, T, -1))
+        if M > 64 and gu.use_kernel and gu.g_idx is None and gu.bias is None and \
+                kernel_choice(M, gu.out_features, gu.in_features, gu._group_size(), tiled=True) == "bgemm" and \
+                gate_up_silu_rows_supported(M, gu.out_features, gu.in_features, gu._group_size()) and \
+                (self._glu_ready() or not torch.cuda.is_current_stream_capturing()):
+            # a prompt on the big-tile GEMM: the same in its epilogue
+            w_t, sz = self._glu_buffers()
+            act = matmul_w4a16_gate_up_silu_rows(n2.reshape(M, -1).contiguous(), w_t, sz,
+                                                 gu._group_size(), gu.out_features)
+            return self.down(act.reshape(B, T, -1))
         return self._down(gu(n2), B, T)
+
+    def _glu_ready(self) -> bool:
+        """Whether the copies of ``_glu_buffers`` exist for the present weights."""
+        cache = getattr(self, "_glu", None)
+        return cache is not None and cache[0] == self.gate_up.fused._stamp()
 
     def _glu_buffers(self):
         """Tiled and group-major copies of the fused gate/up weight with its rows

@@ -345,6 +345,33 @@ def matmul_w4a16_gate_up_silu(x: torch.Tensor, w_tiled: torch.Tensor,
     return out
 
 
+def gate_up_silu_rows_supported(M: int, N: int, K: int, group_size: int) -> bool:
+    """Whether ``matmul_w4a16_gate_up_silu_rows`` runs this shape."""
+    return bool(_lib.lib().pmi_gate_up_silu_rows_supported(M, N, K, group_size))
+
+
+def matmul_w4a16_gate_up_silu_rows(x: torch.Tensor, w_tiled: torch.Tensor,
+                                   sz_gm: tuple[torch.Tensor, torch.Tensor], group_size: int,
+                                   N: int) -> torch.Tensor:
+    """``matmul_w4a16_gate_up_silu`` for many activation rows (prefill): the
+    activation formed in the big-tile GEMM's epilogue, bit for bit the fused
+    matmul followed by ``silu_mul``."""
+    if not x.is_cuda:
+        raise RuntimeError("matmul_w4a16_gate_up_silu_rows requires HIP (cuda) tensors.")
+    assert x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous(), \
+        "x must be a contiguous float16 [M, K] tensor"
+    M, K = x.shape
+    s_gm, z_gm = sz_gm
+    dev = x.device
+    out = torch.empty(M, N // 2, device=dev, dtype=torch.float16)
+    with _DeviceGuard(dev):
+        _lib.check(_lib.lib().pmi_matmul_w4a16_gate_up_silu_rows(
+            _aligned16(x).data_ptr(), _aligned16(w_tiled).data_ptr(), _aligned16(s_gm).data_ptr(),
+            z_gm.data_ptr(), out.data_ptr(), M, N, K, group_size, _stream_handle(dev)),
+            "pmi_matmul_w4a16_gate_up_silu_rows")
+    return out
+
+
 def matmul_w4a16_rmsnorm(x: torch.Tensor, residual: torch.Tensor | None, norm_weight: torch.Tensor,
                          eps: float, packed_weight: torch.Tensor, scales: torch.Tensor,
                          zeros_u8: torch.Tensor, group_size: int):

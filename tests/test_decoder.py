@@ -661,3 +661,26 @@ def test_rope_kv_wide_equals_the_pairwise_kernel(B, T, H, KV, L):
     for a, b in zip(*got):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
     assert got[0][1].abs().sum() > 0
+
+
+@pytest.mark.parametrize("M,F,K", [(2048, 4096, 1536), (1537, 4128, 2048), (129, 14336, 1536)])
+def test_gate_up_silu_rows_equals_matmul_then_silu(M, F, K):
+    """silu(gate) * up in the big-tile GEMM's epilogue (one and two wave groups per
+    workgroup, a last panel that ends inside a band, ragged rows) against the fused
+    matmul followed by silu_mul: the same bits."""
+    from pare_amd.kernels import (gate_up_silu_rows_supported, glu_row_order, kernel_choice,
+                                  matmul_w4a16_gate_up_silu_rows)
+
+    N = 2 * F
+    assert gate_up_silu_rows_supported(M, N, K, 128) and kernel_choice(M, N, K, 128, tiled=True) == "bgemm"
+    g = torch.Generator(device=DEV).manual_seed(M)
+    wk = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8, device=DEV)
+    s = torch.rand(N, K // 128, generator=g, device=DEV) * 0.01 + 1e-3
+    z = torch.randint(0, 16, (N, K // 128), generator=g, dtype=torch.uint8, device=DEV)
+    x = torch.randn(M, K, generator=g, device=DEV).half()
+    y = P.matmul_w4a16(x, wk, s, z, 128, sz_gm=P.sz_group_major(s, z), w_tiled=P.tile_w4a16(wk, 128))
+    idx = glu_row_order(F, DEV)
+    got = matmul_w4a16_gate_up_silu_rows(x, P.tile_w4a16(wk[idx].contiguous(), 128),
+                                         P.sz_group_major(s[idx].contiguous(), z[idx].contiguous()), 128, N)
+    assert torch.equal(got.view(torch.int16), silu_mul(y).view(torch.int16))
+    assert not gate_up_silu_rows_supported(64, N, K, 128) and not gate_up_silu_rows_supported(M, N, K, 64)
