@@ -1,8 +1,8 @@
 // GPTQ producer kernels (pare/schemes/gptq.py:156-263): the sequential column
 // loop of one 128-column block, the per-group scale/zero of the dynamic-group
-// (desc_act) variant, and the final un-permute + INT4 pack. The Cholesky chain
-// and the lazy update of the columns right of a block are library work
-// (rocSOLVER / rocBLAS through torch) driven by the host.
+// (desc_act) variant, the final un-permute + INT4 pack, and the diagonal blocks
+// of the inverse Hessian's factor. The rest of the factor and the lazy update of
+// the columns right of a block are GEMMs driven by the host.
 //
 // Rows are independent in GPTQ: row n's codes depend only on W[n, :] and the
 // shared factor C.

@@ -7,6 +7,8 @@ kernels for gfx950 behind libpare_amd.so:
     (w4a16_gemv.hip), HBM-bandwidth bound;
   - M <= 16 with the activations within 64 KiB of LDS and group size % 128 == 0:
     the skinny MFMA kernel (w4a16_skinny.hip);
+  - many rows: the big-tile GEMM (w4a16_bgemm.hip), from the tiled copy or the
+    kernel layout, every group size that is 32, 64 or a multiple of 128, and bf16;
   - otherwise: MFMA GEMM (w4a16_gemm.hip) for group sizes that are multiples
     of 128 and K % 256 == 0, or the GEMV four activation rows at a time.
 There is no CPU or PyTorch fallback: every call runs the HIP library or raises.
@@ -191,8 +193,9 @@ def matmul_w4a16_bf16(
     which ``matmul_w4a16`` keeps. Here the bf16 values are used as they are
     (fp32 accumulation, y rounded to bf16): with ``w_tiled`` and ``sz_gm`` and
     no ``perm``, the row counts an fp16 call runs on the tiled GEMM's 16-row
-    blocks take its bf16 variant; the rest run on the GEMV, four activation
-    rows per launch. Other arguments as for ``matmul_w4a16``."""
+    blocks take its bf16 variant; more than 24 rows (11 on large layers) run on
+    the big-tile GEMM (N % 4 == 0, K % 128 == 0), the rest on the GEMV, four
+    activation rows per launch. Other arguments as for ``matmul_w4a16``."""
     if not x.is_cuda:
         raise RuntimeError("matmul_w4a16_bf16 requires HIP (cuda) tensors.")
     assert x.is_contiguous(), "x must be contiguous"
