@@ -97,22 +97,29 @@ def _validated_zero_tensor(zeros: torch.Tensor) -> tuple[torch.Tensor, int]:
 
 
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
+# Workspaces that a captured graph was given, by address: its replays read them
+# after an eager call has needed a larger one.
+_CAPTURED_WORKSPACES: dict[int, torch.Tensor] = {}
 
 
 def _workspace(dev: torch.device, stream: int, nbytes: int) -> torch.Tensor | None:
     """Zero-filled scratch for the GEMM's split-K counters/partials and the
     act_order gather, one per (device, stream): launches on one stream are
-    ordered, so they can share it (each call leaves it zero-filled again)."""
+    ordered, so they can share it (each call leaves it zero-filled again). Sizes
+    are powers of two, so those kept for graphs add up to less than the latest."""
     if nbytes == 0:
         return None
     key = (dev.index if dev.index is not None else torch.cuda.current_device(), stream)
     ws = _WORKSPACES.get(key)
+    capturing = torch.cuda.is_current_stream_capturing()
     if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
+        ws = torch.zeros(1 << max(nbytes - 1, (1 << 20) - 1).bit_length(), dtype=torch.uint8, device=dev)
         # under capture the zero fill is only recorded: such a workspace belongs
         # to the graph, whose replays fill it, and is not kept for eager calls
-        if not torch.cuda.is_current_stream_capturing():
+        if not capturing:
             _WORKSPACES[key] = ws
+    elif capturing:
+        _CAPTURED_WORKSPACES[ws.data_ptr()] = ws
     return ws
 
 

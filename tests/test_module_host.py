@@ -3,6 +3,9 @@ fusion rules (pare/layers/linear.py:40-99 buffer contract)."""
 
 from __future__ import annotations
 
+import gc
+import weakref
+
 import pytest
 import torch
 
@@ -46,3 +49,32 @@ def test_fused_rejects_mismatched_layers():
         P.FusedQuantizedLinear([_ql(64, 256, g_idx=g), _ql(64, 256)])
     with pytest.raises(ValueError, match="at least one"):
         P.FusedQuantizedLinear([])
+
+
+def test_workspace_of_a_captured_graph_outlives_a_larger_one(monkeypatch):
+    """A graph's replays read the workspace its calls were captured with, also
+    after an eager call on the same stream needed more."""
+    from pare_amd import kernels as KN
+
+    monkeypatch.setattr(KN, "_WORKSPACES", {})
+    monkeypatch.setattr(KN, "_CAPTURED_WORKSPACES", {}, raising=False)
+    capturing = False
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    dev = torch.device("cpu", 0)
+
+    def held(nbytes):
+        ref = weakref.ref(KN._workspace(dev, 7, nbytes))
+        gc.collect()
+        return ref
+
+    first = held(1 << 20)
+    assert first() is not None
+    second = held((1 << 20) + 1)               # no graph was given the first one
+    assert first() is None and second() is not None
+    capturing = True
+    assert held(1 << 20)() is second()
+    own = held(1 << 24)                        # belongs to the graph's own pool
+    capturing = False
+    third = held(1 << 22)
+    assert own() is None
+    assert third() is not second() and second() is not None
