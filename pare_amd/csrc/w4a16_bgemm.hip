@@ -637,10 +637,7 @@ BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16)
   // workgroups of one group.
   c.kg = tiles <= cus && units > 1 ? 2 : 1;
   // Fewer tiles than half the CUs: split K, at least kMinUnits units a split.
-#ifndef KMINU
-#define KMINU 4
-#endif
-  constexpr int kMinUnits = KMINU;
+  constexpr int kMinUnits = 4;
   int64_t splits = 1;
   if (2 * tiles <= cus) {
     splits = cus / tiles;
