@@ -38,7 +38,7 @@
 // Group sizes. KSG = 32-column k-steps per scale group inside a unit: 4 (group
 // sizes that are multiples of 128), 2 (64) and 1 (32), whose scales and zero
 // points are staged in LDS as well (fewer activation rows make room: MT = 7
-// and 6).
+// and 6). Few rows take MT = 4 (bgemm_config).
 //
 // bf16 (BF). gfx950 has no packed bf16 subtract: B is 128 + q (exact) and a
 // group's sum starts from -(128 + z) * sum x instead of 0; the row sums
@@ -619,6 +619,13 @@ hipError_t launch_shape(const BgemmArgs& a, const BgemmConfig& c, bool rm, hipSt
   return hipGetLastError();
 }
 
+// MT: the most activation tiles whose LDS fits twice on a CU, or 4 (bgemm_config).
+template <int MT, int KSG, bool BF>
+hipError_t launch_mt(const BgemmArgs& a, const BgemmConfig& c, bool rm, hipStream_t stream) {
+  if (c.mt == 4) return launch_shape<4, KSG, BF>(a, c, rm, stream);
+  return launch_shape<MT, KSG, BF>(a, c, rm, stream);
+}
+
 }  // namespace
 
 BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16) {
@@ -628,6 +635,13 @@ BgemmConfig bgemm_config(int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16)
   if (gs != 32 && gs != 64 && gs % 128 != 0) return c;
   if (M * K * 2 >= (1ll << 31) || ((N + 63) / 64) * 64 * (K / 2) >= (1ll << 31)) return c;
   c.mt = gs == 32 ? 6 : (gs == 64 || bf16) ? 7 : 8;
+  // Up to 64 rows, and where 128 rows take two of the taller tiles: tiles of 64
+  // rows, whose products and folds are not spent on rows that are not there (us,
+  // tall tiles / these): bf16 14336 x 4096 at M = 32 / 64 / 120 26.5 / 27.7 / 43.2
+  // against 21.6 / 22.4 / 34.1; 28672 x 4096 at M = 113 66.0 against 49.2; gs 64 at
+  // M = 40 / 128 31.7 / 47.4 against 26.9 / 38.4; gs 32, 4096 x 14336 at M = 100 40.5
+  // against 33.4.
+  if (M <= 64 || (M > 16 * c.mt && M <= 128)) c.mt = 4;
   const int64_t bands = ((N + 63) / 64 + 3) / 4;
   const int64_t gm = (M + 16 * c.mt - 1) / (16 * c.mt);
   const int64_t cus = device_cu_count(), tiles = bands * gm, units = K / 128;
@@ -704,11 +718,9 @@ hipError_t launch_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w_
   a.splits = c.splits;
   a.chunk = c.chunk;
   a.sums_ld = c.sums_ld;
-  if (gs == 32)
-    return bf16 ? launch_shape<6, 1, true>(a, c, rm, stream) : launch_shape<6, 1, false>(a, c, rm, stream);
-  if (gs == 64)
-    return bf16 ? launch_shape<7, 2, true>(a, c, rm, stream) : launch_shape<7, 2, false>(a, c, rm, stream);
-  return bf16 ? launch_shape<7, 4, true>(a, c, rm, stream) : launch_shape<8, 4, false>(a, c, rm, stream);
+  if (gs == 32) return bf16 ? launch_mt<6, 1, true>(a, c, rm, stream) : launch_mt<6, 1, false>(a, c, rm, stream);
+  if (gs == 64) return bf16 ? launch_mt<7, 2, true>(a, c, rm, stream) : launch_mt<7, 2, false>(a, c, rm, stream);
+  return bf16 ? launch_mt<7, 4, true>(a, c, rm, stream) : launch_mt<8, 4, false>(a, c, rm, stream);
 }
 
 }  // namespace pmi

@@ -67,6 +67,13 @@ def _bound(x, w_hat, s, gs, bf16):
     (97, 900, 160 * 4, 32, False, False, False), (12, 16644, 2048, 32, False, False, True),
     # fp16 with the copies: K split over few tiles, from M N K = 1.8e10
     (643, 2060, 14336, 128, False, True, False), (1153, 4096, 4096, 128, False, True, True),
+    # the edges of the 64-row tile: up to 64 rows, and past one taller tile up to 128
+    (64, 772, 1536, 128, True, True, False), (65, 772, 1536, 128, True, True, False),
+    (48, 4100, 1536, 32, True, True, True), (64, 516, 1536, 64, True, True, False),
+    (113, 260, 1152, 64, True, False, False), (128, 516, 640, 32, True, False, False),
+    (129, 516, 640, 32, True, False, False), (128, 17156, 256, 128, True, False, False),
+    (64, 516, 1408, 128, False, False, False), (65, 516, 1408, 128, False, False, False),
+    (128, 516, 1152, 64, False, False, False), (97, 4100, 14336, 32, False, True, False),
     # fp16 without the copies, large enough to leave the register-streamed GEMM
     (769, 5636, 4096, 128, False, False, False),
 ])
