@@ -504,12 +504,13 @@ size_t tgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size
 // time, the tiled GEMM 64 rows at a time, or the register-streamed GEMM.
 
 // GEMV calls of many rows: no other kernel reads the shape's group size or
-// column count, or x is bf16. The GEMV streams the weights once per four rows
-// (4096 x 4096: 5.3 us each), the big-tile GEMM takes 15-25 us for any few rows
-// (gs 64, M = 16 / 32: 22 / 43 against 21 / 22 us; 14336 x 4096, M = 16: 61
-// against 30).
+// column count, or x is bf16. The GEMV streams the weights once per four rows,
+// the big-tile GEMM's 64-row tiles take the same time for any few rows (us, GEMV /
+// big-tile): 4096 x 4096 gs 64 at M = 16 / 20 / 28 22 / 27.5 / 38 against 19.3; bf16
+// 20 / 26 / 36 against 21; 1024 x 4096 gs 64 bf16 19 / 23 / 32 against 19.3; 14336 x
+// 4096 gs 64 at M = 13 / 24 50 / 85 against 27; 4096 x 14336 bf16 50 / 84 against 30.
 bool bgemm_over_gemv(int64_t M, int64_t N, int64_t K) {
-  return M > 24 || (M >= 12 && N * K >= (1ll << 25));
+  return M > 16 || (M >= 12 && N * K >= (1ll << 25));
 }
 
 // Group sizes 32 and 64 on the tiled copy, past 64 rows (tiled GEMM / big-tile,

@@ -67,6 +67,8 @@ def _bound(x, w_hat, s, gs, bf16):
     (97, 900, 160 * 4, 32, False, False, False), (12, 16644, 2048, 32, False, False, True),
     # fp16 with the copies: K split over few tiles, from M N K = 1.8e10
     (643, 2060, 14336, 128, False, True, False), (1153, 4096, 4096, 128, False, True, True),
+    # the fewest rows that leave the GEMV
+    (17, 516, 1536, 128, True, False, False), (17, 1028, 1152, 64, False, False, True),
     # the edges of the 64-row tile: up to 64 rows, and past one taller tile up to 128
     (64, 772, 1536, 128, True, True, False), (65, 772, 1536, 128, True, True, False),
     (48, 4100, 1536, 32, True, True, True), (64, 516, 1536, 64, True, True, False),
