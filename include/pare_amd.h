@@ -354,6 +354,12 @@ PMI_API size_t pmi_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K, int64
 PMI_API size_t pmi_matmul_best_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size,
                                                int has_perm);
 
+/* *id: the id of the graph capture that stream is part of, unique in the process,
+ * or 0 where it is not capturing. A workspace that a captured call uses must be
+ * that graph's alone: its replays run on any stream, beside other calls on the
+ * one it was captured on. Host-only. No reference counterpart. */
+PMI_API int pmi_stream_capture_id(void* stream, uint64_t* id);
+
 /* Full dequantised weight W_hat[N,K] in the original column order, cast to
  * out_dtype (PMI_F16 / PMI_BF16 with round-to-nearest-even, or PMI_F32).
  * layout PMI_LAYOUT_STORAGE: idx (nullable) is g_idx int32 [K], the group of

@@ -659,6 +659,16 @@ size_t pmi_matmul_best_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t 
   return big > base ? big : base;
 }
 
+int pmi_stream_capture_id(void* stream, uint64_t* id) {
+  const char* fn = "pmi_stream_capture_id";
+  if (!id) return fail(PMI_ERR_INVALID, "%s: null id", fn);
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long n = 0;
+  const hipError_t e = hipStreamGetCaptureInfo((hipStream_t)stream, &status, &n);
+  *id = e == hipSuccess && status == hipStreamCaptureStatusActive ? n : 0;
+  return from_hip(e, fn);
+}
+
 int pmi_sz_group_major(const float* scales, const void* zeros, int zero_dtype, float* scales_gm,
                        uint8_t* zeros_gm, int32_t* bad_count, int64_t N, int64_t G,
                        void* stream) {

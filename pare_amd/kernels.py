@@ -16,6 +16,8 @@ There is no CPU or PyTorch fallback: every call runs the HIP library or raises.
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -96,30 +98,49 @@ def _validated_zero_tensor(zeros: torch.Tensor) -> tuple[torch.Tensor, int]:
     return z, _lib.PMI_F32
 
 
+# The split-K counters at the head of a workspace: all of it that has to be zero
+# before a call (and is again after it).
+_COUNTER_BYTES = 64 * 1024
+
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
-# Workspaces that a captured graph was given, by address: its replays read them
-# after an eager call has needed a larger one.
-_CAPTURED_WORKSPACES: dict[int, torch.Tensor] = {}
+# (capture id, workspace) of the last capture on a stream
+_CAPTURE_WORKSPACES: dict[tuple[int, int], tuple[int, torch.Tensor]] = {}
+
+
+def _new_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
+    ws = torch.empty(1 << max(nbytes - 1, (1 << 20) - 1).bit_length(), dtype=torch.uint8, device=dev)
+    ws[:_COUNTER_BYTES].zero_()
+    return ws
+
+
+def _capture_id(stream: int) -> int:
+    n = ctypes.c_uint64()
+    _lib.check(_lib.lib().pmi_stream_capture_id(stream, ctypes.byref(n)), "pmi_stream_capture_id")
+    return n.value
 
 
 def _workspace(dev: torch.device, stream: int, nbytes: int) -> torch.Tensor | None:
-    """Zero-filled scratch for the GEMM's split-K counters/partials and the
+    """Scratch for the GEMMs' split-K counters and partials, row sums and the
     act_order gather, one per (device, stream): launches on one stream are
-    ordered, so they can share it (each call leaves it zero-filled again). Sizes
-    are powers of two, so those kept for graphs add up to less than the latest."""
+    ordered, so they can share it. A graph is replayed on any stream, beside
+    eager calls on the one it was captured on: each capture has a workspace of
+    its own, shared by its calls on a stream, in the graph's memory pool (which
+    keeps the memory; the tensor is let go at the next call after the capture)
+    and with its counters cleared by the graph itself."""
     if nbytes == 0:
         return None
     key = (dev.index if dev.index is not None else torch.cuda.current_device(), stream)
+    if torch.cuda.is_current_stream_capturing():
+        capture = _capture_id(stream)
+        last, ws = _CAPTURE_WORKSPACES.get(key, (None, None))
+        if last != capture or ws.numel() < nbytes:
+            ws = _new_workspace(dev, nbytes)
+            _CAPTURE_WORKSPACES[key] = (capture, ws)
+        return ws
+    _CAPTURE_WORKSPACES.pop(key, None)
     ws = _WORKSPACES.get(key)
-    capturing = torch.cuda.is_current_stream_capturing()
     if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(1 << max(nbytes - 1, (1 << 20) - 1).bit_length(), dtype=torch.uint8, device=dev)
-        # under capture the zero fill is only recorded: such a workspace belongs
-        # to the graph, whose replays fill it, and is not kept for eager calls
-        if not capturing:
-            _WORKSPACES[key] = ws
-    elif capturing:
-        _CAPTURED_WORKSPACES[ws.data_ptr()] = ws
+        ws = _WORKSPACES[key] = _new_workspace(dev, nbytes)
     return ws
 
 

@@ -191,3 +191,32 @@ def test_bgemm_in_a_captured_graph(bf16, gs):
         torch.cuda.synchronize()
         assert torch.equal(y.view(torch.int16), want.view(torch.int16)), k
         assert torch.equal(eager.view(torch.int16), want.view(torch.int16)), k
+
+
+def test_bgemm_graph_replays_beside_eager_work_on_its_capture_stream():
+    """A graph captured on a stream whose eager calls use the same scratch,
+    replayed on another stream while that one is busy: row sums and partial
+    tiles of the two stay apart."""
+    M, N, K, gs = 130, 1028, 4096, 128
+    wk, s, zu8, _, _ = _case(N, K, gs, 9, False)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    x, xe = (torch.randn(M, K, device=DEV, generator=g).bfloat16() for _ in range(2))
+    want, want_e = (P.matmul_w4a16_bf16(v, wk, s, zu8, gs) for v in (x, xe))
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        P.matmul_w4a16_bf16(xe, wk, s, zu8, gs)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        y = P.matmul_w4a16_bf16(x, wk, s, zu8, gs)
+    for _ in range(4):
+        got, eager = [], []
+        for _ in range(16):
+            with torch.cuda.stream(side):
+                eager.append(P.matmul_w4a16_bf16(xe, wk, s, zu8, gs))
+            graph.replay()
+            got.append(y.clone())
+        torch.cuda.synchronize()
+        for a, b in zip(got, eager):
+            assert torch.equal(a.view(torch.int16), want.view(torch.int16))
+            assert torch.equal(b.view(torch.int16), want_e.view(torch.int16))

@@ -51,30 +51,33 @@ def test_fused_rejects_mismatched_layers():
         P.FusedQuantizedLinear([])
 
 
-def test_workspace_of_a_captured_graph_outlives_a_larger_one(monkeypatch):
-    """A graph's replays read the workspace its calls were captured with, also
-    after an eager call on the same stream needed more."""
+def test_workspaces_of_captures_and_eager_calls_are_apart(monkeypatch):
+    """A graph's replays may run beside eager calls on the stream it was captured
+    on, and beside another graph captured there: none of them shares a workspace,
+    and what a capture holds is let go once it has ended."""
     from pare_amd import kernels as KN
 
-    monkeypatch.setattr(KN, "_WORKSPACES", {})
-    monkeypatch.setattr(KN, "_CAPTURED_WORKSPACES", {}, raising=False)
-    capturing = False
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
-    dev = torch.device("cpu", 0)
+    capture = 0
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capture != 0)
+    monkeypatch.setattr(KN, "_capture_id", lambda stream: capture, raising=False)
+    dev, stream = torch.device("cpu", 0), 0x7007
 
-    def held(nbytes):
-        ref = weakref.ref(KN._workspace(dev, 7, nbytes))
-        gc.collect()
-        return ref
-
-    first = held(1 << 20)
-    assert first() is not None
-    second = held((1 << 20) + 1)               # no graph was given the first one
-    assert first() is None and second() is not None
-    capturing = True
-    assert held(1 << 20)() is second()
-    own = held(1 << 24)                        # belongs to the graph's own pool
-    capturing = False
-    third = held(1 << 22)
-    assert own() is None
-    assert third() is not second() and second() is not None
+    eager = KN._workspace(dev, stream, 1 << 20)
+    capture = 11
+    first = KN._workspace(dev, stream, 1 << 20)
+    assert first is not eager and KN._workspace(dev, stream, 1 << 19) is first
+    assert first[:64 * 1024].eq(0).all()
+    larger = KN._workspace(dev, stream, (1 << 20) + 1)
+    assert larger is not first and KN._workspace(dev, stream, 1 << 20) is larger
+    capture = 12
+    second = KN._workspace(dev, stream, 1 << 20)
+    capture = 0
+    assert KN._workspace(dev, stream, 1 << 20) is eager
+    assert len({t.data_ptr() for t in (eager, first, larger, second)}) == 4
+    refs = [weakref.ref(t) for t in (first, larger, second)]
+    del first, larger, second
+    gc.collect()
+    assert all(r() is None for r in refs)
+    # another eager call of the stream that needs more replaces its workspace
+    grown = KN._workspace(dev, stream, (1 << 20) + 1)
+    assert grown is not eager and KN._workspace(dev, stream, 1 << 20) is grown
