@@ -17,6 +17,7 @@ There is no CPU or PyTorch fallback: every call runs the HIP library or raises.
 from __future__ import annotations
 
 import ctypes
+import threading
 
 import torch
 
@@ -102,9 +103,19 @@ def _validated_zero_tensor(zeros: torch.Tensor) -> tuple[torch.Tensor, int]:
 # before a call (and is again after it).
 _COUNTER_BYTES = 64 * 1024
 
-_WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
-# (capture id, workspace) of the last capture on a stream
-_CAPTURE_WORKSPACES: dict[tuple[int, int], tuple[int, torch.Tensor]] = {}
+
+class _Workspaces(threading.local):
+    """One thread's workspaces by (device, stream), given back when it ends: a
+    call of several launches (row sums or gather, product, sum of the partials)
+    is not one step for another thread that launches on the same stream."""
+
+    def __init__(self):
+        self.eager: dict[tuple[int, int], torch.Tensor] = {}
+        # (capture id, workspace) of the last capture on a stream
+        self.captured: dict[tuple[int, int], tuple[int, torch.Tensor]] = {}
+
+
+_workspaces = _Workspaces()
 
 
 def _new_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
@@ -121,8 +132,8 @@ def _capture_id(stream: int) -> int:
 
 def _workspace(dev: torch.device, stream: int, nbytes: int) -> torch.Tensor | None:
     """Scratch for the GEMMs' split-K counters and partials, row sums and the
-    act_order gather, one per (device, stream): launches on one stream are
-    ordered, so they can share it. A graph is replayed on any stream, beside
+    act_order gather, one per thread, device and stream: a thread's launches on a
+    stream are ordered, so they can share it. A graph is replayed on any stream, beside
     eager calls on the one it was captured on: each capture has a workspace of
     its own, shared by its calls on a stream, in the graph's memory pool (which
     keeps the memory; the tensor is let go at the next call after the capture)
@@ -132,15 +143,15 @@ def _workspace(dev: torch.device, stream: int, nbytes: int) -> torch.Tensor | No
     key = (dev.index if dev.index is not None else torch.cuda.current_device(), stream)
     if torch.cuda.is_current_stream_capturing():
         capture = _capture_id(stream)
-        last, ws = _CAPTURE_WORKSPACES.get(key, (None, None))
+        last, ws = _workspaces.captured.get(key, (None, None))
         if last != capture or ws.numel() < nbytes:
             ws = _new_workspace(dev, nbytes)
-            _CAPTURE_WORKSPACES[key] = (capture, ws)
+            _workspaces.captured[key] = (capture, ws)
         return ws
-    _CAPTURE_WORKSPACES.pop(key, None)
-    ws = _WORKSPACES.get(key)
+    _workspaces.captured.pop(key, None)
+    ws = _workspaces.eager.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = _WORKSPACES[key] = _new_workspace(dev, nbytes)
+        ws = _workspaces.eager[key] = _new_workspace(dev, nbytes)
     return ws
 
 

@@ -4,6 +4,7 @@ fusion rules (pare/layers/linear.py:40-99 buffer contract)."""
 from __future__ import annotations
 
 import gc
+import threading
 import weakref
 
 import pytest
@@ -81,3 +82,28 @@ def test_workspaces_of_captures_and_eager_calls_are_apart(monkeypatch):
     # another eager call of the stream that needs more replaces its workspace
     grown = KN._workspace(dev, stream, (1 << 20) + 1)
     assert grown is not eager and KN._workspace(dev, stream, 1 << 20) is grown
+
+
+def test_threads_on_one_stream_have_workspaces_of_their_own(monkeypatch):
+    """Two threads that launch on the same stream: the launches of their calls
+    may interleave, so neither works in the other's scratch, and a thread that
+    has ended keeps none."""
+    from pare_amd import kernels as KN
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    dev, stream = torch.device("cpu", 0), 0x7107
+    mine = KN._workspace(dev, stream, 1 << 20)
+    other = []
+
+    def work():
+        ws = KN._workspace(dev, stream, 1 << 20)
+        assert KN._workspace(dev, stream, 1 << 20) is ws
+        other.append((ws.data_ptr(), weakref.ref(ws)))
+
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    assert other and other[0][0] != mine.data_ptr()
+    gc.collect()
+    assert other[0][1]() is None
+    assert KN._workspace(dev, stream, 1 << 20) is mine
