@@ -97,6 +97,14 @@ py::object matmul(const at::Tensor& x, const at::Tensor& w, const at::Tensor& sc
     if (c == 5 || c == 6) return py::none();
   }
 
+  const size_t need = g_workspace(M, N, K, gs, perm ? 1 : 0);
+  at::Tensor ws;
+  if (need) {
+    ws = workspace_fn(need).cast<at::Tensor>();
+    if (!plain(ws) || ws.device() != dev) return py::none();
+  }
+  // other threads run meanwhile: a launch waits where the stream's queue is full
+  std::optional<py::gil_scoped_release> unlocked(std::in_place);
   at::Tensor xc = native || in == at::kHalf ? x : x.to(at::kHalf);
   xc = xc.contiguous();
   if (reinterpret_cast<uintptr_t>(xc.const_data_ptr()) % 16) xc = xc.clone();
@@ -104,12 +112,6 @@ py::object matmul(const at::Tensor& x, const at::Tensor& w, const at::Tensor& sc
   shape.back() = N;
   at::Tensor y = at::empty(shape, at::TensorOptions().dtype(xc.scalar_type()).device(dev));
 
-  const size_t need = g_workspace(M, N, K, gs, perm ? 1 : 0);
-  at::Tensor ws;
-  if (need) {
-    ws = workspace_fn(need).cast<at::Tensor>();
-    if (!plain(ws) || ws.device() != dev) return py::none();
-  }
   const int code = native ? kBf16 : kF16;
   const int rc = g_matmul(xc.const_data_ptr(), code, static_cast<const uint8_t*>(w.const_data_ptr()),
                           static_cast<const float*>(scales.const_data_ptr()), zeros.const_data_ptr(), kU8,
@@ -117,10 +119,10 @@ py::object matmul(const at::Tensor& x, const at::Tensor& w, const at::Tensor& sc
                           use_tiled ? ptr<uint8_t>(w_tiled) : nullptr, y.mutable_data_ptr(), code, M, N, K, gs,
                           need ? ws.mutable_data_ptr() : nullptr, need ? (size_t)ws.numel() : 0,
                           reinterpret_cast<void*>(stream));
-  if (rc != 0) return py::none();
-  if (y.scalar_type() != in) y = y.to(in);
-  if (bias) y = y + *bias;
-  return py::cast(y);
+  if (rc == 0 && y.scalar_type() != in) y = y.to(in);
+  if (rc == 0 && bias) y = y + *bias;
+  unlocked.reset();
+  return rc == 0 ? py::cast(y) : py::none();
 }
 
 }  // namespace

@@ -4,10 +4,13 @@ not."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
 import pare_amd as P
+from pare_amd import _lib
 from pare_amd import kernels as KN
 from pare_amd.config import QuantConfig
 from pare_amd.linear import QuantizedLinear
@@ -115,3 +118,24 @@ def test_vmap_and_subclasses_are_not_read_as_plain_tensors():
     assert torch.equal(torch.as_tensor(layer(sub)).as_subclass(torch.Tensor), want)
     with pytest.raises(RuntimeError):
         torch.vmap(layer)(x)
+
+
+def test_other_threads_run_during_the_library_call():
+    """The library's entry points are called without the interpreter lock, as
+    ctypes calls them: a launch on a full queue waits, and what it waits for may
+    need the lock (a host callback in Python). In the place of the matmul: whether
+    the calling thread holds it, where 0 counts as success."""
+    layer = _layer(256, 1536, 128)
+    x = torch.randn(4, 1536, device=DEV).half()
+    layer(x)
+    L, ext = _lib.lib(), _lib.host()
+    fns = [ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in (
+        "pmi_matmul_w4a16", "pmi_matmul_kernel_choice", "pmi_matmul_best_workspace_bytes")]
+    held = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    try:
+        ext.bind(held, *fns[1:])
+        y = layer._forward_host(x)
+    finally:
+        ext.bind(*fns)
+    assert y is not None and y.shape == (4, 256)
+    assert torch.equal(layer._forward_host(x), layer._forward_kernel(x))
