@@ -557,7 +557,7 @@ size_t ws_sz_bytes(int64_t N, int64_t K, int64_t gs) {
 }
 
 // Workspace that lets the big-tile GEMM take the calls above and split K (with
-// less they run as they would without it, or unsplit).
+// less they run as they would without it, or unsplit: bgemm_fits).
 size_t bgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t gs, bool has_perm) {
   if (M < 12) return 0;
   size_t need = 0;
@@ -574,14 +574,41 @@ size_t bgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t gs, bool h
   return need ? pmi::kWsCounterBytes + (has_perm ? pmi::ws_perm_bytes(M, K) : 0) + need : 0;
 }
 
+// Few tiles whose K split has no room in the workspace, in the place of the GEMV:
+// one workgroup per tile takes 2.6-3.0 us per two units of K (4.1 with tiles taller
+// than 64 rows), the GEMV a launch per four rows (us, GEMV / unsplit): 512 x 14336
+// at M = 17 / 128 / 256 21.4 / 146 / 295 against 147 / 151 / 198; 4096 x 4096 at M =
+// 17 / 32 / 48 24 / 41 / 61 against 46 / 48 / 48; 14336 x 4096 at M = 17 62 against 47;
+// gs 64 within 15 % of these.
+bool unsplit_over_gemv(int64_t M, int64_t N, int64_t K, const pmi::BgemmConfig& b) {
+  const double steps = (double)((K / 128 + 1) / 2);
+  return (double)((M + 3) / 4) * (3.3 + (double)(N * K) / 7.5e6) > 5.0 + steps * (b.mt == 4 ? 2.9 : 4.1);
+}
+
+// The kernel whose call the big-tile GEMM takes: none (its own choice), the GEMV,
+// or another GEMM.
+enum class Takes { kNone, kGemv, kGemm };
+
+// Whether a workspace of ws_bytes, of which the first `off` bytes are spoken for,
+// lets the big-tile GEMM run such a call well. Unsplit, the tiled GEMM or the
+// register-streamed GEMM is faster than the tiles that ask for a split (tiled / unsplit,
+// us, gs 64): 4096 x 14336 at M = 65 / 301 53 / 139 against 186 / 188; 1024 x 14336 at
+// M = 1024 135 against 182; 14336 x 4096 at M = 192 39 against 58.
+bool bgemm_fits(Takes takes, size_t off, size_t ws_bytes, int64_t M, int64_t N, int64_t K,
+                const pmi::BgemmConfig& b) {
+  const size_t need = off + b.ws_sums;
+  if (need > pmi::kWsCounterBytes && ws_bytes < need) return false;
+  if (takes == Takes::kNone || b.splits == 1 || ws_bytes >= need + b.ws_split) return true;
+  return takes == Takes::kGemv && unsplit_over_gemv(M, N, K, b);
+}
+
 // Runs the big-tile GEMM: X[:, perm] gathered first with act_order, the
 // group-major copies made in the workspace where gm is false. *ran = false (and
-// nothing launched) when the workspace is too small for what it cannot do
-// without.
+// nothing launched) when the workspace is too small (bgemm_fits).
 hipError_t run_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w, const float* scales,
                      const void* zeros, int zero_u8, const float* scales_gm, const uint8_t* zeros_gm,
                      const int32_t* perm, void* y, int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16,
-                     void* workspace, size_t ws_bytes, hipStream_t s, bool* ran) {
+                     void* workspace, size_t ws_bytes, hipStream_t s, Takes takes, bool* ran) {
   const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, gs, bf16);
   const bool gm = scales_gm && zeros_gm;
   size_t off = pmi::kWsCounterBytes;
@@ -589,7 +616,7 @@ hipError_t run_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w, co
   if (perm) off += pmi::ws_perm_bytes(M, K);
   const size_t sz_off = off;
   if (!gm) off += ws_sz_bytes(N, K, gs);
-  *ran = off + b.ws_sums == pmi::kWsCounterBytes || (workspace && ws_bytes >= off + b.ws_sums);
+  *ran = bgemm_fits(takes, off, ws_bytes, M, N, K, b);
   if (!*ran) return hipSuccess;
   uint8_t* ws = (uint8_t*)workspace;
   if (perm) {
@@ -745,7 +772,7 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
     if (!forced && aligned(y, 8) && use_bgemm(1, true, gm && w_tiled, gm, M, N, K, group_size)) {
       bool ran = false;
       const hipError_t e = run_bgemm(x, gm ? w_tiled : nullptr, w, scales, zeros, zu8, scales_gm, zeros_gm, perm, y,
-                                     M, N, K, group_size, true, workspace, workspace_bytes, s, &ran);
+                                     M, N, K, group_size, true, workspace, workspace_bytes, s, Takes::kGemv, &ran);
       if (ran) return from_hip(e, fn);
     }
     const uint16_t* xp = (const uint16_t*)x;
@@ -794,7 +821,7 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
                   "N %% 4 == 0, K %% 512 == 0, K >= 1536, group_size %% 128 == 0 and M * K < 2^30", fn);
     bool ran = false;
     const hipError_t e = run_bgemm(x, w_tiled, w, scales, zeros, zu8, scales_gm, zeros_gm, perm, y, M, N, K,
-                                   group_size, false, workspace, workspace_bytes, s, &ran);
+                                   group_size, false, workspace, workspace_bytes, s, Takes::kNone, &ran);
     if (!ran)
       return fail(PMI_ERR_UNSUPPORTED, "%s: the big-tile GEMM with perm needs a workspace of "
                   "pmi_matmul_workspace_bytes() bytes", fn);
@@ -804,7 +831,8 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
   if (!forced && aligned(y, 8) && use_bgemm(choice, false, has_tiled, gm, M, N, K, group_size)) {
     bool ran = false;
     const hipError_t e = run_bgemm(x, has_tiled ? w_tiled : nullptr, w, scales, zeros, zu8, scales_gm, zeros_gm,
-                                   perm, y, M, N, K, group_size, false, workspace, workspace_bytes, s, &ran);
+                                   perm, y, M, N, K, group_size, false, workspace, workspace_bytes, s,
+                                   choice == 1 ? Takes::kGemv : Takes::kGemm, &ran);
     if (ran) return from_hip(e, fn);
   }
   if (choice == 5) {

@@ -166,6 +166,46 @@ def test_bgemm_split_without_its_workspace_runs_elsewhere():
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("M,N,K,gs,bf16,copies,kernel", [
+    (301, 4096, 14336, 64, False, True, "tgemm"), (65, 4096, 14336, 64, False, True, "tgemm"),
+    (193, 4100, 4096, 32, False, True, "tgemm"), (1024, 1024, 18944, 128, False, False, "gemm64"),
+    (17, 512, 14336, 128, True, False, "gemv"), (28, 4096, 4096, 64, False, False, "gemv"),
+])
+def test_bgemm_leaves_few_tiles_whose_split_has_no_room(M, N, K, gs, bf16, copies, kernel):
+    """With the workspace that pmi_matmul_workspace_bytes reports, or one that
+    holds all but the partial tiles, such calls run on the kernel that took them
+    before (same bits), through the C ABI: unsplit they would occupy 2-80 CUs."""
+    L = _lib.lib()
+    g = torch.Generator(device=DEV).manual_seed(4)
+    wk = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8, device=DEV)
+    s = torch.rand(N, K // gs, generator=g, device=DEV) * 0.01 + 1e-3
+    z = torch.randint(0, 16, (N, K // gs), generator=g, dtype=torch.uint8, device=DEV)
+    dtype, code = (torch.bfloat16, _lib.PMI_BF16) if bf16 else (torch.float16, _lib.PMI_F16)
+    x = torch.randn(M, K, generator=g, device=DEV).to(dtype)
+    gm = P.sz_group_major(s, z) if copies else None
+    wt = P.tile_w4a16(wk, gs) if copies else None
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def call(nbytes):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=DEV) if nbytes else None
+        y = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+        rc = L.pmi_matmul_w4a16(x.data_ptr(), code, wk.data_ptr(), s.data_ptr(), z.data_ptr(), _lib.PMI_U8,
+                                None, None, gm[0].data_ptr() if gm else None, gm[1].data_ptr() if gm else None,
+                                wt.data_ptr() if copies else None, y.data_ptr(), code, M, N, K, gs,
+                                ws.data_ptr() if nbytes else None, nbytes, stream)
+        assert rc == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        return y
+
+    base = L.pmi_matmul_workspace_bytes(M, N, K, gs, 0)
+    print(f"[case] no room M={M} N={N} K={K} gs={gs} bf16={bf16} base={base}", flush=True)
+    assert L.pmi_matmul_best_workspace_bytes(M, N, K, gs, 0) > max(base, 2 << 20)
+    for nbytes in (base, 2 << 20):
+        with force_kernel(kernel):
+            want = call(nbytes)
+        assert torch.equal(call(nbytes).view(torch.int16), want.view(torch.int16)), nbytes
+
+
 @pytest.mark.parametrize("bf16,gs", [(True, 128), (False, 64)])
 def test_bgemm_in_a_captured_graph(bf16, gs):
     """A captured call that no eager call warmed up (its workspace then belongs
