@@ -437,8 +437,11 @@ PMI_API int pmi_gptq_pack(const uint8_t* codes, const int32_t* inv_perm, uint8_t
  * scales_gm and zeros_gm), and an act_order perm. */
 #define PMI_CHOICE_TILED 1
 #define PMI_CHOICE_PERM  2
+/* of pmi_matmul_route only: scales_gm and zeros_gm without the tiled copy */
+#define PMI_CHOICE_GM    4
 
-/* Which kernel pmi_matmul_w4a16 would run for this shape: 1 = split-K GEMV,
+/* The kernel for an fp16 call of this shape before the big-tile rules that also look
+ * at the copies and the workspace (pmi_matmul_route applies those): 1 = split-K GEMV,
  * 2 = MFMA GEMM (group_size % 128 == 0 and K % 256 == 0), 3 = skinny MFMA
  * kernel (M <= 16), 4 = register-streamed MFMA GEMM (group_size == 128,
  * K % 512 == 0), 5 = tiled-weight MFMA GEMM (K % 512 == 0, K >= 1536,
@@ -447,13 +450,22 @@ PMI_API int pmi_gptq_pack(const uint8_t* codes, const int32_t* inv_perm, uint8_t
  * as well, up to 16 rows it gathers X[:, perm] itself when M (2K + 16) + 4K
  * bytes fit its LDS, which widens where it wins), 6 = the tiled GEMM's
  * big-tile variant (same buffers; many activation rows, group_size % 128 ==
- * 0: 256 weight rows x 128 activation rows per workgroup, B formed as
- * fp16((q - z) * s) as the reference dequantises; with PMI_CHOICE_PERM
- * X[:, perm] is gathered into the workspace first). flags 0 and 1 keep the
- * meaning of the former has_tiled argument. Host-only; no reference
+ * 0: 256 weight rows x up to 128 activation rows per tile, exact products x (q - z)
+ * summed in fp32 and scaled once per group; with PMI_CHOICE_PERM X[:, perm] is
+ * gathered into the workspace first). Calls reported as 1, 2, 4 or 5 run on 6 as
+ * well where that is faster and the workspace has room (group sizes 32 and 64,
+ * no tiled copy). flags 0 and 1 keep the meaning of the former has_tiled argument. Host-only; no reference
  * counterpart (the reference has one Triton kernel). */
 PMI_API int pmi_matmul_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t group_size,
                                      int flags);
+
+/* The kernel (numbered as above) that runs a pmi_matmul_w4a16 call of x_dtype (PMI_F16 or
+ * PMI_BF16) with the buffers that flags name, a workspace of workspace_bytes bytes
+ * and y 8-byte aligned, or a negative PMI_ERR_ code. 6 reads the tiled copy where
+ * there is one (PMI_CHOICE_TILED), else the kernel layout. Host-only; no reference
+ * counterpart. */
+PMI_API int pmi_matmul_route(int64_t M, int64_t N, int64_t K, int64_t group_size, int x_dtype, int flags,
+                             size_t workspace_bytes);
 
 /* The K ranges the tiled-weight GEMM (kernel 5) splits this shape into when
  * the call has a workspace of pmi_matmul_workspace_bytes() bytes. Up to 16

@@ -23,7 +23,7 @@ PMI_ERR_HIP = -3
 PMI_ERR_NO_DEVICE = -4
 
 PMI_F16, PMI_BF16, PMI_F32, PMI_U8 = 0, 1, 2, 3
-PMI_CHOICE_TILED, PMI_CHOICE_PERM = 1, 2
+PMI_CHOICE_TILED, PMI_CHOICE_PERM, PMI_CHOICE_GM = 1, 2, 4
 PMI_LAYOUT_STORAGE, PMI_LAYOUT_KERNEL = 0, 1
 
 _ERR_NAMES = {
@@ -67,6 +67,7 @@ SIGNATURES = {
     "pmi_dequant_w4a16": (_i, [_vp, _i, _vp, _vp, _i, _vp, _vp, _i, _i64, _i64, _i64, _vp]),
     "pmi_rtn_quantize": (_i, [_vp, _i, _vp, _vp, _vp, _i64, _i64, _i64, _i, _vp]),
     "pmi_matmul_kernel_choice": (_i, [_i64, _i64, _i64, _i64, _i]),
+    "pmi_matmul_route": (_i, [_i64, _i64, _i64, _i64, _i, _i, ctypes.c_size_t]),
     "pmi_tgemm_splits": (_i, [_i64, _i64, _i64, _i64, _i]),
     "pmi_matmul_w4a16_gate_up_silu": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "pmi_gate_up_silu_supported": (_i, [_i64, _i64, _i64, _i64]),

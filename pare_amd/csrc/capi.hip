@@ -589,49 +589,104 @@ bool unsplit_over_gemv(int64_t M, int64_t N, int64_t K, const pmi::BgemmConfig& 
 // or another GEMM.
 enum class Takes { kNone, kGemv, kGemm };
 
-// Whether a workspace of ws_bytes, of which the first `off` bytes are spoken for,
-// lets the big-tile GEMM run such a call well. Unsplit, the tiled GEMM or the
-// register-streamed GEMM is faster than the tiles that ask for a split (tiled / unsplit,
-// us, gs 64): 4096 x 14336 at M = 65 / 301 53 / 139 against 186 / 188; 1024 x 14336 at
-// M = 1024 135 against 182; 14336 x 4096 at M = 192 39 against 58.
-bool bgemm_fits(Takes takes, size_t off, size_t ws_bytes, int64_t M, int64_t N, int64_t K,
-                const pmi::BgemmConfig& b) {
-  const size_t need = off + b.ws_sums;
-  if (need > pmi::kWsCounterBytes && ws_bytes < need) return false;
-  if (takes == Takes::kNone || b.splits == 1 || ws_bytes >= need + b.ws_split) return true;
-  return takes == Takes::kGemv && unsplit_over_gemv(M, N, K, b);
+// One call as the kernels' limits see it.
+struct Call {
+  int64_t M, N, K, gs;
+  bool bf16;
+  bool tiled;  // w_tiled, with the group-major copies
+  bool gm;     // the group-major copies
+  bool perm;
+  bool y8;     // y is 8-byte aligned
+  size_t ws;   // workspace bytes
+};
+
+// Workspace in front of the big-tile GEMM's row sums and partial tiles: the
+// counters, X[:, perm], and the group-major copies of a caller without them.
+size_t bgemm_offset(const Call& c) {
+  return pmi::kWsCounterBytes + (c.perm ? pmi::ws_perm_bytes(c.M, c.K) : 0) +
+         (c.gm ? 0 : ws_sz_bytes(c.N, c.K, c.gs));
+}
+
+// Whether the workspace lets the big-tile GEMM run the call well. Unsplit, the tiled
+// GEMM or the register-streamed GEMM is faster than the tiles that ask for a split
+// (tiled / unsplit, us, gs 64): 4096 x 14336 at M = 65 / 301 53 / 139 against 186 / 188;
+// 1024 x 14336 at M = 1024 135 against 182; 14336 x 4096 at M = 192 39 against 58.
+bool bgemm_fits(const Call& c, Takes takes) {
+  const pmi::BgemmConfig b = pmi::bgemm_config(c.M, c.N, c.K, c.gs, c.bf16);
+  const size_t need = bgemm_offset(c) + b.ws_sums;
+  if (need > pmi::kWsCounterBytes && c.ws < need) return false;
+  if (takes == Takes::kNone || b.splits == 1 || c.ws >= need + b.ws_split) return true;
+  return takes == Takes::kGemv && unsplit_over_gemv(c.M, c.N, c.K, b);
+}
+
+// The tiled GEMM's bf16 variant.
+bool bf16_on_tgemm(const Call& c) {
+  return c.tiled && c.N % 4 == 0 && !c.perm && c.y8 && pmi::tgemm_bf16_supported(c.M, c.N, c.K, c.gs);
+}
+
+// MFMA GEMM with act_order: X[:, perm] fits the workspace.
+bool gemm_perm_fits(const Call& c) {
+  return !c.perm || !pmi::gemm_supported(c.K, c.gs) ||
+         c.ws >= pmi::gemm_workspace_bytes(c.M, c.N, c.K, c.gs, true) -
+                     pmi::gemm_config(c.M, c.N, c.K, c.gs, true).ws_split;
+}
+
+// The kernel that runs a call (numbered as pmi_matmul_kernel_choice numbers them).
+int route(const Call& c) {
+  const auto choice = [&](int flags) { return pmi_matmul_kernel_choice(c.M, c.N, c.K, c.gs, flags); };
+  if (c.bf16) {
+    // the rows an fp16 call would run on the tiled GEMM's 16-row blocks take its
+    // bf16 variant, many rows the big-tile GEMM, the rest the GEMV
+    if (bf16_on_tgemm(c) && choice(PMI_CHOICE_TILED) == 5) return 5;
+    return c.y8 && use_bgemm(1, true, c.tiled, c.gm, c.M, c.N, c.K, c.gs) && bgemm_fits(c, Takes::kGemv) ? 6 : 1;
+  }
+  // the tiled GEMM reads the tiled weights and the group-major scale/zero copies;
+  // its epilogue (both variants) stores up to four fp16 outputs (8 bytes) per lane
+  const bool tiled = c.tiled && c.N % 4 == 0;
+  const int perm = c.perm ? PMI_CHOICE_PERM : 0;
+  int k = choice((tiled ? PMI_CHOICE_TILED : 0) | perm);
+  if ((k == 5 || k == 6) && !c.y8) k = choice(perm);
+  if (k == 6) {
+    // without the workspace of its K split the big-tile GEMM leaves such a call
+    // to the kernel it would run on without the tiled copy
+    const pmi::BgemmConfig b = pmi::bgemm_config(c.M, c.N, c.K, c.gs);
+    const size_t room = pmi::kWsCounterBytes + (perm ? pmi::ws_perm_bytes(c.M, c.K) : 0) + b.ws_split;
+    if ((int64_t)b.n_bands * b.grid_m * 4 >= 3 * pmi::device_cu_count() || c.ws >= room) return 6;
+    k = choice(perm);
+  }
+  if (c.y8 && use_bgemm(k, false, tiled, c.gm, c.M, c.N, c.K, c.gs) &&
+      bgemm_fits(c, k == 1 ? Takes::kGemv : Takes::kGemm))
+    return 6;
+  // act_order: without room for X[:, perm] the tiled GEMM leaves rows that it does
+  // not gather itself to the others, and the MFMA GEMM leaves them to the GEMV
+  if (k == 5 && perm && !pmi::tgemm_gather_supported(c.M, c.K) &&
+      c.ws < pmi::kWsCounterBytes + pmi::ws_perm_bytes(c.M, c.K))
+    k = choice(0);
+  return k == 2 && !gemm_perm_fits(c) ? 1 : k;
 }
 
 // Runs the big-tile GEMM: X[:, perm] gathered first with act_order, the
-// group-major copies made in the workspace where gm is false. *ran = false (and
-// nothing launched) when the workspace is too small (bgemm_fits).
-hipError_t run_bgemm(const void* x, const uint8_t* w_tiled, const uint8_t* w, const float* scales,
+// group-major copies made in the workspace where there are none.
+hipError_t run_bgemm(const Call& c, const void* x, const uint8_t* w_tiled, const uint8_t* w, const float* scales,
                      const void* zeros, int zero_u8, const float* scales_gm, const uint8_t* zeros_gm,
-                     const int32_t* perm, void* y, int64_t M, int64_t N, int64_t K, int64_t gs, bool bf16,
-                     void* workspace, size_t ws_bytes, hipStream_t s, Takes takes, bool* ran) {
-  const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, gs, bf16);
-  const bool gm = scales_gm && zeros_gm;
-  size_t off = pmi::kWsCounterBytes;
-  const size_t perm_off = off;
-  if (perm) off += pmi::ws_perm_bytes(M, K);
-  const size_t sz_off = off;
-  if (!gm) off += ws_sz_bytes(N, K, gs);
-  *ran = bgemm_fits(takes, off, ws_bytes, M, N, K, b);
-  if (!*ran) return hipSuccess;
-  uint8_t* ws = (uint8_t*)workspace;
+                     const int32_t* perm, void* y, void* workspace, hipStream_t s) {
+  uint8_t* at = (uint8_t*)workspace + pmi::kWsCounterBytes;
   if (perm) {
-    if (hipError_t e = pmi::launch_gather_cols(x, perm, ws + perm_off, M, K, s); e != hipSuccess) return e;
-    x = ws + perm_off;
+    if (hipError_t e = pmi::launch_gather_cols(x, perm, at, c.M, c.K, s); e != hipSuccess) return e;
+    x = at;
+    at += pmi::ws_perm_bytes(c.M, c.K);
   }
-  if (!gm) {
-    float* s_out = (float*)(ws + sz_off);
-    uint8_t* z_out = ws + sz_off + pmi::ws_align((size_t)N * (K / gs) * 4);
-    if (hipError_t e = pmi::launch_sz_group_major(scales, zeros, zero_u8, 0, s_out, z_out, nullptr, N, K / gs, s);
+  if (!c.gm) {
+    float* s_out = (float*)at;
+    uint8_t* z_out = at + pmi::ws_align((size_t)c.N * (c.K / c.gs) * 4);
+    if (hipError_t e =
+            pmi::launch_sz_group_major(scales, zeros, zero_u8, 0, s_out, z_out, nullptr, c.N, c.K / c.gs, s);
         e != hipSuccess)
       return e;
     scales_gm = s_out, zeros_gm = z_out;
   }
-  return pmi::launch_bgemm(x, w_tiled, w, scales_gm, zeros_gm, y, M, N, K, gs, bf16, workspace, ws_bytes, off, s);
+  return pmi::launch_bgemm(x, c.tiled && c.N % 4 == 0 ? w_tiled : nullptr, w, scales_gm, zeros_gm, y, c.M, c.N, c.K,
+                           c.gs, c.bf16, workspace, c.ws, bgemm_offset(c), s);
 }
 
 size_t other_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size, int has_perm) {
@@ -656,6 +711,20 @@ size_t other_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size
 }
 
 }  // namespace
+
+int pmi_matmul_route(int64_t M, int64_t N, int64_t K, int64_t group_size, int x_dtype, int flags,
+                     size_t workspace_bytes) {
+  const char* fn = "pmi_matmul_route";
+  if (int rc = check_shape(N, K, group_size, fn)) return rc;
+  if (M < 1 || N < 1) return fail(PMI_ERR_INVALID, "%s: need M >= 1 and N >= 1", fn);
+  if (x_dtype != PMI_F16 && x_dtype != PMI_BF16)
+    return fail(PMI_ERR_UNSUPPORTED, "%s: x must be fp16 or bf16 (got %d)", fn, x_dtype);
+  const bool tiled = flags & PMI_CHOICE_TILED;
+  const int forced = g_kernel_override.load();
+  return forced ? forced
+                : route({M, N, K, group_size, x_dtype == PMI_BF16, tiled, tiled || (flags & PMI_CHOICE_GM),
+                         (flags & PMI_CHOICE_PERM) != 0, true, workspace_bytes});
+}
 
 int pmi_tgemm_splits(int64_t M, int64_t N, int64_t K, int64_t group_size, int has_perm) {
   if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || K % group_size != 0 ||
@@ -748,33 +817,26 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
   hipStream_t s = (hipStream_t)stream;
   const int zu8 = zero_dtype == PMI_U8;
   const int forced = g_kernel_override.load();
+  const bool gm = scales_gm && zeros_gm;
+  const Call call{M, N, K, group_size, bf, w_tiled && gm, gm, perm != nullptr, aligned(y, 8), workspace_bytes};
+  const int choice = forced ? forced : route(call);
   if (bf) {
-    // bf16 activations (the native bf16 extension): with the tiled copy, the
-    // rows an fp16 call would run on the tiled GEMM's 16-row blocks (no
-    // act_order) take its bf16 variant; the rest run on the GEMV, four
-    // activation rows per launch, act_order rows gathered into the workspace
-    // first (2-byte elements, as for fp16)
+    // bf16 activations (the native bf16 extension)
     if (forced && forced != 1 && forced != 5)
-      return fail(PMI_ERR_UNSUPPORTED, "%s: bf16 activations run on the GEMV or the tiled GEMM only "
+      return fail(PMI_ERR_UNSUPPORTED, "%s: bf16 activations are forced onto the GEMV or the tiled GEMM only "
                   "(kernel %d forced)", fn, forced);
-    const bool bf_tiled = w_tiled && scales_gm && zeros_gm && N % 4 == 0 && !perm && aligned(y, 8) &&
-                          pmi::tgemm_bf16_supported(M, N, K, group_size);
-    if (forced == 5 && !bf_tiled)
+    if (forced == 5 && !bf16_on_tgemm(call))
       return fail(PMI_ERR_UNSUPPORTED, "%s: the tiled GEMM's bf16 variant needs w_tiled, scales_gm and "
                   "zeros_gm, no perm, y 8-byte aligned, group_size %% 128 == 0 and 16-row blocks", fn);
-    if (bf_tiled && (forced == 5 || (!forced && pmi_matmul_kernel_choice(M, N, K, group_size,
-                                                                         PMI_CHOICE_TILED) == 5)))
+    if (choice == 5)
       return from_hip(pmi::launch_tgemm(x, nullptr, nullptr, w_tiled, scales_gm, zeros_gm, y, M, N,
                                         K, group_size, nullptr, 0, 0, s, true),
                       fn);
-    // many rows: the big-tile GEMM, from the tiled copy where there is one
-    const bool gm = scales_gm && zeros_gm;
-    if (!forced && aligned(y, 8) && use_bgemm(1, true, gm && w_tiled, gm, M, N, K, group_size)) {
-      bool ran = false;
-      const hipError_t e = run_bgemm(x, gm ? w_tiled : nullptr, w, scales, zeros, zu8, scales_gm, zeros_gm, perm, y,
-                                     M, N, K, group_size, true, workspace, workspace_bytes, s, Takes::kGemv, &ran);
-      if (ran) return from_hip(e, fn);
-    }
+    if (choice == 6)
+      return from_hip(run_bgemm(call, x, w_tiled, w, scales, zeros, zu8, scales_gm, zeros_gm, perm, y, workspace, s),
+                      fn);
+    // the GEMV, four activation rows per launch, act_order rows gathered into the
+    // workspace first (2-byte elements, as for fp16)
     const uint16_t* xp = (const uint16_t*)x;
     if (perm) {
       if (workspace_bytes < pmi::kWsCounterBytes + pmi::ws_perm_bytes(M, K))
@@ -796,44 +858,19 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
     }
     return ok();
   }
-  // the tiled GEMM reads the tiled weights and the group-major scale/zero copies
-  const bool has_tiled = w_tiled && scales_gm && zeros_gm && N % 4 == 0;
-  int choice = pmi_matmul_kernel_choice(
-      M, N, K, group_size, (has_tiled ? PMI_CHOICE_TILED : 0) | (perm ? PMI_CHOICE_PERM : 0));
-  // the tiled GEMM's epilogue (both variants) stores up to four fp16 outputs
-  // (8 bytes) per lane
-  if ((choice == 5 || choice == 6) && !aligned(y, 8)) {
-    if (forced) return fail(PMI_ERR_INVALID, "%s: the tiled GEMM needs y 8-byte aligned", fn);
-    choice = pmi_matmul_kernel_choice(M, N, K, group_size, perm ? PMI_CHOICE_PERM : 0);
-  }
-  // without the workspace of its K split the big-tile GEMM leaves such a call
-  // to the kernel it would run on without the tiled copy
-  if (choice == 6 && !forced) {
-    const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, group_size);
-    const size_t room = pmi::kWsCounterBytes + (perm ? pmi::ws_perm_bytes(M, K) : 0) + b.ws_split;
-    if ((int64_t)b.n_bands * b.grid_m * 4 < 3 * pmi::device_cu_count() && workspace_bytes < room)
-      choice = pmi_matmul_kernel_choice(M, N, K, group_size, perm ? PMI_CHOICE_PERM : 0);
-  }
+  const bool has_tiled = call.tiled && N % 4 == 0;
+  if ((forced == 5 || forced == 6) && !call.y8)
+    return fail(PMI_ERR_INVALID, "%s: the tiled GEMM needs y 8-byte aligned", fn);
   if (choice == 6) {
-    if (!has_tiled || !pmi::tgemm_supported(M, N, K, group_size) || group_size % 128 != 0 ||
-        !pmi::bgemm_config(M, N, K, group_size).ok)
+    if (forced && (!has_tiled || !pmi::tgemm_supported(M, N, K, group_size) || group_size % 128 != 0 ||
+                   !pmi::bgemm_config(M, N, K, group_size).ok))
       return fail(PMI_ERR_UNSUPPORTED, "%s: the big-tile GEMM needs w_tiled, scales_gm and zeros_gm, "
                   "N %% 4 == 0, K %% 512 == 0, K >= 1536, group_size %% 128 == 0 and M * K < 2^30", fn);
-    bool ran = false;
-    const hipError_t e = run_bgemm(x, w_tiled, w, scales, zeros, zu8, scales_gm, zeros_gm, perm, y, M, N, K,
-                                   group_size, false, workspace, workspace_bytes, s, Takes::kNone, &ran);
-    if (!ran)
+    if (!bgemm_fits(call, Takes::kNone))
       return fail(PMI_ERR_UNSUPPORTED, "%s: the big-tile GEMM with perm needs a workspace of "
                   "pmi_matmul_workspace_bytes() bytes", fn);
-    return from_hip(e, fn);
-  }
-  const bool gm = scales_gm && zeros_gm;
-  if (!forced && aligned(y, 8) && use_bgemm(choice, false, has_tiled, gm, M, N, K, group_size)) {
-    bool ran = false;
-    const hipError_t e = run_bgemm(x, has_tiled ? w_tiled : nullptr, w, scales, zeros, zu8, scales_gm, zeros_gm,
-                                   perm, y, M, N, K, group_size, false, workspace, workspace_bytes, s,
-                                   choice == 1 ? Takes::kGemv : Takes::kGemm, &ran);
-    if (ran) return from_hip(e, fn);
+    return from_hip(run_bgemm(call, x, w_tiled, w, scales, zeros, zu8, scales_gm, zeros_gm, perm, y, workspace, s),
+                    fn);
   }
   if (choice == 5) {
     if (!has_tiled || !pmi::tgemm_supported(M, N, K, group_size))
@@ -857,20 +894,13 @@ int pmi_matmul_w4a16(const void* x, int x_dtype, const uint8_t* w, const float* 
                                         pmi::kWsCounterBytes + pmi::ws_perm_bytes(M, K), s),
                       fn);
     }
-    if (forced) return fail(PMI_ERR_UNSUPPORTED, "%s: forced tiled GEMM with perm needs a "
-                            "workspace of pmi_matmul_workspace_bytes() bytes", fn);
-    choice = pmi_matmul_kernel_choice(M, N, K, group_size, 0);
+    return fail(PMI_ERR_UNSUPPORTED, "%s: forced tiled GEMM with perm needs a "
+                "workspace of pmi_matmul_workspace_bytes() bytes", fn);
   }
-  // act_order on the GEMM gathers X[:, perm] into the workspace; without one
-  // the automatic choice falls back to the GEMV.
-  const bool perm_fits = !perm || !pmi::gemm_supported(K, group_size) ||
-                         workspace_bytes >= pmi::gemm_workspace_bytes(M, N, K, group_size, true) -
-                                                pmi::gemm_config(M, N, K, group_size, true).ws_split;
-  if (choice == 2 && !perm_fits) {
-    if (forced) return fail(PMI_ERR_UNSUPPORTED, "%s: forced MFMA GEMM with perm needs a workspace "
-                            "of pmi_matmul_workspace_bytes() bytes", fn);
-    choice = 1;
-  }
+  // act_order on the GEMM gathers X[:, perm] into the workspace
+  if (choice == 2 && !gemm_perm_fits(call))
+    return fail(PMI_ERR_UNSUPPORTED, "%s: forced MFMA GEMM with perm needs a workspace "
+                "of pmi_matmul_workspace_bytes() bytes", fn);
   if (choice == 4 && !pmi::gemm64_supported(M, K, group_size))
     return fail(PMI_ERR_UNSUPPORTED, "%s: forced register-streamed GEMM needs group_size == 128 "
                 "and M*K*2 < 2^31", fn);

@@ -581,11 +581,34 @@ class force_kernel:
 def kernel_choice(M: int, N: int, K: int, group_size: int, tiled: bool = False,
                   perm: bool = False) -> str:
     """'gemv', 'gemm', 'skinny', 'gemm64', 'tgemm' or 'bgemm' (the tiled GEMM's
-    big-tile variant): the kernel matmul_w4a16 runs for this shape (``tiled``: the
-    caller passes the tiled weight copy; ``perm``: an act_order permutation)."""
+    big-tile variant): the kernel for an fp16 call of this shape before the rules
+    that look at the other copies and the workspace as well, and may move it to
+    'bgemm' (``kernel_route``). ``tiled``: the caller passes the tiled weight copy;
+    ``perm``: an act_order permutation."""
     flags = (_lib.PMI_CHOICE_TILED if tiled else 0) | (_lib.PMI_CHOICE_PERM if perm else 0)
-    c = _lib.lib().pmi_matmul_kernel_choice(M, N, K, group_size, flags)
-    return {1: "gemv", 2: "gemm", 3: "skinny", 4: "gemm64", 5: "tgemm", 6: "bgemm"}[c]
+    return _KERNELS[_lib.lib().pmi_matmul_kernel_choice(M, N, K, group_size, flags)]
+
+
+_KERNELS = {1: "gemv", 2: "gemm", 3: "skinny", 4: "gemm64", 5: "tgemm", 6: "bgemm"}
+
+
+def kernel_route(M: int, N: int, K: int, group_size: int, dtype: torch.dtype = torch.float16,
+                 tiled: bool = False, perm: bool = False, gm: bool = False,
+                 workspace: int | None = None) -> str:
+    """The kernel that runs a matmul_w4a16 (or, ``dtype`` bfloat16,
+    matmul_w4a16_bf16) call. ``tiled``: with the tiled and group-major copies;
+    ``gm``: with the latter only; ``workspace``: its bytes, by default what
+    the Python layer gives the call."""
+    L = _lib.lib()
+    if workspace is None:
+        workspace = L.pmi_matmul_best_workspace_bytes(M, N, K, group_size, int(perm))
+    flags = ((_lib.PMI_CHOICE_TILED if tiled else 0) | (_lib.PMI_CHOICE_PERM if perm else 0)
+             | (_lib.PMI_CHOICE_GM if gm else 0))
+    code = {torch.float16: _lib.PMI_F16, torch.bfloat16: _lib.PMI_BF16}[dtype]
+    k = L.pmi_matmul_route(M, N, K, group_size, code, flags, workspace)
+    if k < 0:
+        _lib.check(k, "pmi_matmul_route")
+    return _KERNELS[k]
 
 
 def tgemm_splits(M: int, N: int, K: int, group_size: int, perm: bool = False) -> int:

@@ -274,3 +274,35 @@ def test_error_message_is_thread_local(L):
 def test_pmi_error_maps_to_runtime_error():
     with pytest.raises(RuntimeError, match="PMI_ERR_INVALID"):
         _lib.call("pmi_repack_int4_for_kernel", FAKE, FAKE * 2, None, 8, 200, 128, None)
+
+
+@pytest.mark.parametrize("M,N,K,gs,bf16,flags,ws,kernel", [
+    # as pmi_matmul_kernel_choice has it
+    (1, 4096, 4096, 128, False, 1, 0, 1), (16, 4096, 4096, 128, False, 1, 0, 5),
+    (2048, 4096, 4096, 128, False, 1, 0, 6), (128, 4096, 4096, 128, False, 0, 0, 4),
+    (16, 4096, 4096, 128, True, 1, 0, 5), (16, 4096, 4096, 128, True, 0, 0, 1),
+    # the big-tile GEMM from what the GEMV, the tiled and the register-streamed GEMM take
+    (64, 4096, 4096, 128, True, 0, -1, 6), (64, 4096, 4096, 64, False, 0, -1, 6),
+    (301, 4096, 14336, 64, False, 1, -1, 6), (769, 5636, 4096, 128, False, 0, -1, 6),
+    (512, 4096, 4096, 256, True, 1, -1, 6), (512, 4096, 4096, 256, True, 0, -1, 1),
+    (384, 14336, 4096, 128, False, 0, -1, 6), (512, 14336, 4096, 128, False, 4, 0, 6),
+    (225, 2060, 2048, 256, True, 3, -1, 6), (130, 516, 1152, 64, True, 2, -1, 6),
+    # ... which need room: for the row sums or group-major copies, and for the split
+    (64, 4096, 4096, 128, True, 0, 0, 1), (64, 4096, 4096, 64, False, 0, 0, 1),
+    (301, 4096, 14336, 64, False, 1, 0, 5), (643, 2060, 14336, 128, False, 1, 0, 4),
+    (1024, 1024, 18944, 128, False, 0, 8 << 20, 4),
+    # unsplit in the GEMV's place where its launches cost more
+    (17, 512, 14336, 128, True, 4, 1 << 20, 1), (256, 512, 14336, 128, True, 4, 1 << 20, 6),
+    (32, 4096, 4096, 64, False, 0, 2 << 20, 1), (64, 4096, 4096, 64, False, 0, 2 << 20, 6),
+])
+def test_matmul_route(L, M, N, K, gs, bf16, flags, ws, kernel):
+    """The kernel that runs a call, workspace included (-1: all it can use)."""
+    if ws < 0:
+        ws = L.pmi_matmul_best_workspace_bytes(M, N, K, gs, int(bool(flags & 2)))
+    assert L.pmi_matmul_route(M, N, K, gs, _lib.PMI_BF16 if bf16 else _lib.PMI_F16, flags, ws) == kernel
+
+
+def test_matmul_route_rejects_what_the_matmul_rejects(L):
+    assert L.pmi_matmul_route(1, 64, 100, 64, _lib.PMI_F16, 0, 0) == _lib.PMI_ERR_INVALID
+    assert L.pmi_matmul_route(0, 64, 128, 64, _lib.PMI_F16, 0, 0) == _lib.PMI_ERR_INVALID
+    assert L.pmi_matmul_route(1, 64, 128, 64, _lib.PMI_F32, 0, 0) == _lib.PMI_ERR_UNSUPPORTED
