@@ -24,18 +24,21 @@ using MatmulFn = int (*)(const void*, int, const uint8_t*, const float*, const v
                          int64_t, int64_t, int64_t, void*, size_t, void*);
 using ChoiceFn = int (*)(int64_t, int64_t, int64_t, int64_t, int);
 using WorkspaceFn = size_t (*)(int64_t, int64_t, int64_t, int64_t, int);
+using RouteFn = int (*)(int64_t, int64_t, int64_t, int64_t, int, int, size_t);
 
 MatmulFn g_matmul = nullptr;
 ChoiceFn g_choice = nullptr;
 WorkspaceFn g_workspace = nullptr;
+RouteFn g_route = nullptr;
 
 constexpr int kF16 = 0, kBf16 = 1, kU8 = 3;  // PMI_F16, PMI_BF16, PMI_U8
-constexpr int kChoiceTiled = 1, kChoicePerm = 2;
+constexpr int kChoiceTiled = 1, kChoicePerm = 2, kChoiceGm = 4;
 
-void bind(uintptr_t matmul, uintptr_t choice, uintptr_t workspace) {
+void bind(uintptr_t matmul, uintptr_t choice, uintptr_t workspace, uintptr_t route) {
   g_matmul = reinterpret_cast<MatmulFn>(matmul);
   g_choice = reinterpret_cast<ChoiceFn>(choice);
   g_workspace = reinterpret_cast<WorkspaceFn>(workspace);
+  g_route = reinterpret_cast<RouteFn>(route);
 }
 
 bool plain(const at::Tensor& t) {
@@ -96,8 +99,10 @@ py::object matmul(const at::Tensor& x, const at::Tensor& w, const at::Tensor& sc
     const int c = g_choice(M, N, K, gs, kChoiceTiled | (perm ? kChoicePerm : 0));
     if (c == 5 || c == 6) return py::none();
   }
-
   const size_t need = g_workspace(M, N, K, gs, perm ? 1 : 0);
+  if (!w_tiled && build_tiled && native && !perm &&
+      g_route(M, N, K, gs, kBf16, kChoiceTiled, need) != g_route(M, N, K, gs, kBf16, s_gm ? kChoiceGm : 0, need))
+    return py::none();
   at::Tensor ws;
   if (need) {
     ws = workspace_fn(need).cast<at::Tensor>();

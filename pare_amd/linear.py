@@ -21,7 +21,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .config import QuantConfig, is_int4, kernel_group_size
-from .kernels import host_matmul, kernel_choice, matmul_w4a16, matmul_w4a16_bf16
+from .kernels import host_matmul, kernel_choice, kernel_route, matmul_w4a16, matmul_w4a16_bf16
 from .pack import (dequantize_int4, perm_from_g_idx, perm_u16, repack_int4_for_kernel,
                    sz_group_major, tile_w4a16, tiled_supported, zeros_to_u8)
 
@@ -143,18 +143,24 @@ class QuantizedLinear(nn.Module):
             cache = self._kernel_cache
         return self._packed_weight_kernel, cache[1], cache[2], cache[3]
 
-    def _tiled_buffer(self, w_kernel: torch.Tensor, M: int, perm: torch.Tensor | None = None):
+    def _tiled_buffer(self, w_kernel: torch.Tensor, M: int, perm: torch.Tensor | None = None,
+                      bf16: bool = False):
         """Tiled copy of the kernel-layout weight for the tiled-weight GEMM,
         built on the first forward whose row count runs on it (decode-only use
         at one row never pays for it) and kept with the kernel-layout weight
-        (dropped with it when the weights change). Under graph capture a copy
+        (dropped with it when the weights change). ``bf16``: also where a native
+        bf16 call runs on another kernel with the copy (groups of 256 columns and
+        more have no other matrix-core kernel), so that its kernel does not
+        depend on whether an earlier call has built it. Under graph capture a copy
         that does not exist yet is not built (it would only be recorded, and
         eager calls would read it unfilled): the call runs without it."""
         if getattr(self, "_packed_weight_tiled", None) is None:
             if not tiled_supported(self.out_features, self.in_features, self._group_size()):
                 return None
-            if kernel_choice(M, self.out_features, self.in_features, self._group_size(),
-                             tiled=True, perm=perm is not None) not in ("tgemm", "bgemm"):
+            shape = (M, self.out_features, self.in_features, self._group_size())
+            if kernel_choice(*shape, tiled=True, perm=perm is not None) not in ("tgemm", "bgemm") and \
+                    not (bf16 and kernel_route(*shape, torch.bfloat16, tiled=True, perm=perm is not None)
+                         != kernel_route(*shape, torch.bfloat16, gm=True, perm=perm is not None)):
                 return None
             if torch.cuda.is_current_stream_capturing():
                 return None
@@ -200,7 +206,7 @@ class QuantizedLinear(nn.Module):
         orig_shape = x.shape
         if x.dtype == torch.bfloat16 and getattr(self, "native_bf16", False):
             xb = x.reshape(-1, self.in_features).contiguous()
-            w_t = None if perm is not None else self._tiled_buffer(w_k, xb.shape[0])
+            w_t = None if perm is not None else self._tiled_buffer(w_k, xb.shape[0], bf16=True)
             y = matmul_w4a16_bf16(xb, w_k, self.scale, zero_u8, self._group_size(), perm=perm,
                                   perm16=self._perm16, sz_gm=sz_gm, w_tiled=w_t)
             if self.bias is not None:

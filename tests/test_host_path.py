@@ -51,6 +51,24 @@ def test_module_forward_equals_the_general_path(N, K, gs, act_order, dtype, nati
             assert torch.equal(y, want)
 
 
+@pytest.mark.parametrize("N,K,gs,M", [(1024, 4096, 256, 512), (516, 10240, 512, 70), (1024, 4096, 128, 512),
+                                      (512, 2048, 64, 512)])
+def test_native_bf16_does_not_depend_on_earlier_calls(N, K, gs, M):
+    """The kernel (and so the bits) of a native bf16 forward: the same on a fresh
+    layer as after a call of few rows that builds the tiled copy."""
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(3)).bfloat16()
+    outs = []
+    for early in (False, True):
+        layer = _layer(N, K, gs)
+        layer.native_bf16 = True
+        if early:
+            layer(x[:8])
+            assert layer._packed_weight_tiled is not None
+        outs += [layer(x), layer(x)]
+    for y in outs[1:]:
+        assert torch.equal(y.view(torch.int16), outs[0].view(torch.int16))
+
+
 def test_module_inputs_the_host_path_converts_or_leaves():
     layer = _layer(512, 1536, 128)
     x = torch.randn(6, 1536, device=DEV).half()
@@ -130,7 +148,8 @@ def test_other_threads_run_during_the_library_call():
     layer(x)
     L, ext = _lib.lib(), _lib.host()
     fns = [ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in (
-        "pmi_matmul_w4a16", "pmi_matmul_kernel_choice", "pmi_matmul_best_workspace_bytes")]
+        "pmi_matmul_w4a16", "pmi_matmul_kernel_choice", "pmi_matmul_best_workspace_bytes",
+        "pmi_matmul_route")]
     held = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
     try:
         ext.bind(held, *fns[1:])
