@@ -92,16 +92,15 @@ py::object matmul(const at::Tensor& x, const at::Tensor& w, const at::Tensor& sc
   if (s_gm && (!buffer(*s_gm, dev, at::kFloat, N * G, 4) || !buffer(*z_gm, dev, at::kByte, N * G, 4) ||
                s_gm->dim() != 2 || s_gm->size(0) != G || z_gm->dim() != 2 || z_gm->size(0) != G))
     return py::none();
-  // bf16 with act_order runs on kernels that read the kernel layout
-  const bool use_tiled = w_tiled && !(native && perm);
-  if (use_tiled && !buffer(*w_tiled, dev, at::kByte, (N + 63) / 64 * 64 * (K / 2), 16)) return py::none();
+  if (w_tiled && !buffer(*w_tiled, dev, at::kByte, (N + 63) / 64 * 64 * (K / 2), 16)) return py::none();
+  const int act = perm ? kChoicePerm : 0;
   if (!w_tiled && build_tiled && !(native && perm)) {
-    const int c = g_choice(M, N, K, gs, kChoiceTiled | (perm ? kChoicePerm : 0));
+    const int c = g_choice(M, N, K, gs, kChoiceTiled | act);
     if (c == 5 || c == 6) return py::none();
   }
   const size_t need = g_workspace(M, N, K, gs, perm ? 1 : 0);
-  if (!w_tiled && build_tiled && native && !perm &&
-      g_route(M, N, K, gs, kBf16, kChoiceTiled, need) != g_route(M, N, K, gs, kBf16, s_gm ? kChoiceGm : 0, need))
+  if (!w_tiled && build_tiled && native &&
+      g_route(M, N, K, gs, kBf16, kChoiceTiled | act, need) != g_route(M, N, K, gs, kBf16, kChoiceGm | act, need))
     return py::none();
   at::Tensor ws;
   if (need) {
@@ -121,7 +120,7 @@ py::object matmul(const at::Tensor& x, const at::Tensor& w, const at::Tensor& sc
   const int rc = g_matmul(xc.const_data_ptr(), code, static_cast<const uint8_t*>(w.const_data_ptr()),
                           static_cast<const float*>(scales.const_data_ptr()), zeros.const_data_ptr(), kU8,
                           ptr<int32_t>(perm), ptr<uint16_t>(perm16), ptr<float>(s_gm), ptr<uint8_t>(z_gm),
-                          use_tiled ? ptr<uint8_t>(w_tiled) : nullptr, y.mutable_data_ptr(), code, M, N, K, gs,
+                          ptr<uint8_t>(w_tiled), y.mutable_data_ptr(), code, M, N, K, gs,
                           need ? ws.mutable_data_ptr() : nullptr, need ? (size_t)ws.numel() : 0,
                           reinterpret_cast<void*>(stream));
   if (rc == 0 && y.scalar_type() != in) y = y.to(in);

@@ -158,9 +158,13 @@ class QuantizedLinear(nn.Module):
             if not tiled_supported(self.out_features, self.in_features, self._group_size()):
                 return None
             shape = (M, self.out_features, self.in_features, self._group_size())
-            if kernel_choice(*shape, tiled=True, perm=perm is not None) not in ("tgemm", "bgemm") and \
-                    not (bf16 and kernel_route(*shape, torch.bfloat16, tiled=True, perm=perm is not None)
-                         != kernel_route(*shape, torch.bfloat16, gm=True, perm=perm is not None)):
+            act = perm is not None
+            # (the tiled GEMM takes no act_order in bf16)
+            runs = not (bf16 and act) and kernel_choice(*shape, tiled=True, perm=act) in ("tgemm", "bgemm")
+            if not runs and bf16:
+                runs = kernel_route(*shape, torch.bfloat16, tiled=True, perm=act) != \
+                    kernel_route(*shape, torch.bfloat16, gm=True, perm=act)
+            if not runs:
                 return None
             if torch.cuda.is_current_stream_capturing():
                 return None
@@ -206,7 +210,7 @@ class QuantizedLinear(nn.Module):
         orig_shape = x.shape
         if x.dtype == torch.bfloat16 and getattr(self, "native_bf16", False):
             xb = x.reshape(-1, self.in_features).contiguous()
-            w_t = None if perm is not None else self._tiled_buffer(w_k, xb.shape[0], bf16=True)
+            w_t = self._tiled_buffer(w_k, xb.shape[0], perm, bf16=True)
             y = matmul_w4a16_bf16(xb, w_k, self.scale, zero_u8, self._group_size(), perm=perm,
                                   perm16=self._perm16, sz_gm=sz_gm, w_tiled=w_t)
             if self.bias is not None:

@@ -69,6 +69,31 @@ def test_native_bf16_does_not_depend_on_earlier_calls(N, K, gs, M):
         assert torch.equal(y.view(torch.int16), outs[0].view(torch.int16))
 
 
+@pytest.mark.parametrize("gs", [64, 128, 256])
+def test_bf16_act_order_call_reads_the_copies_it_was_given(gs):
+    """A bf16 call with a permutation and the tiled copy: with ``out`` (general
+    path) and without (host extension) it is the same call, on the kernel that
+    the copy allows."""
+    N, K, M = 516, 2048, 225
+    layer = _layer(N, K, gs, act_order=True)
+    layer.native_bf16 = True
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(3)).bfloat16()
+    w, z, perm, sz = layer._kernel_buffers()
+    layer(x[:8])                                     # the GEMV: no copy for it
+    assert layer._packed_weight_tiled is None
+    wt = P.tile_w4a16(w, gs)
+    kw = {"perm": perm, "sz_gm": sz, "w_tiled": wt}
+    assert KN.kernel_route(M, N, K, gs, torch.bfloat16, tiled=True, perm=True) == "bgemm"
+    y = P.matmul_w4a16_bf16(x, w, layer.scale, z, gs, **kw)
+    out = torch.empty_like(y)
+    P.matmul_w4a16_bf16(x, w, layer.scale, z, gs, out=out, **kw)
+    with KN.force_kernel("gemv"):
+        gemv = P.matmul_w4a16_bf16(x, w, layer.scale, z, gs, **kw)
+    for v in (out, layer(x), layer(x)):
+        assert torch.equal(v.view(torch.int16), y.view(torch.int16))
+    assert (y.double() - gemv.double()).norm() <= 4e-3 * gemv.double().norm()
+
+
 def test_module_inputs_the_host_path_converts_or_leaves():
     layer = _layer(512, 1536, 128)
     x = torch.randn(6, 1536, device=DEV).half()
