@@ -145,7 +145,7 @@ def host():
         try:
             from . import _host as ext
         except ImportError as e:
-            raise RuntimeError("pare_amd/_host is not built; run `python -m pare_amd.build`") from e
+            raise RuntimeError(f"pare_amd/_host does not load ({e}); run `python -m pare_amd.build`") from e
         ext.bind(*(ctypes.cast(getattr(handle, fn), ctypes.c_void_p).value for fn in (
             "pmi_matmul_w4a16", "pmi_matmul_kernel_choice", "pmi_matmul_best_workspace_bytes",
             "pmi_matmul_route")))

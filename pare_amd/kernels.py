@@ -49,10 +49,12 @@ class _DeviceGuard:
 
 
 def kernel_available() -> bool:
-    """True if libpare_amd.so is built and the current device is a gfx950 GPU
-    (the probe the reference calls ``triton_available``, matmul_int4.py:246-248)."""
+    """True if libpare_amd.so and the host extension are built and load, and the
+    current device is a gfx950 GPU (the probe the reference calls
+    ``triton_available``, matmul_int4.py:246-248)."""
     try:
         L = _lib.lib()
+        _lib.host()
     except (RuntimeError, OSError):
         return False
     if not torch.cuda.is_available():

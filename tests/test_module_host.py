@@ -107,3 +107,24 @@ def test_threads_on_one_stream_have_workspaces_of_their_own(monkeypatch):
     gc.collect()
     assert other[0][1]() is None
     assert KN._workspace(dev, stream, 1 << 20) is mine
+
+
+def test_kernel_available_needs_the_host_extension(monkeypatch):
+    """matmul_w4a16 raises where the host extension does not load (not built, or
+    built for another torch): the probe then says so."""
+    from types import SimpleNamespace
+
+    from pare_amd import _lib
+    from pare_amd import kernels as KN
+
+    monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(pmi_device_supported=lambda d: 1))
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(_lib, "host", lambda: None)
+    assert KN.kernel_available()
+
+    def missing():
+        raise RuntimeError("not built")
+
+    monkeypatch.setattr(_lib, "host", missing)
+    assert not KN.kernel_available()
