@@ -60,6 +60,32 @@ int check_zero_dtype(int zero_dtype, const char* fn) {
   return PMI_OK;
 }
 
+// The big-tile GEMM with tiles for less than three quarters of the CUs, from M N K =
+// 1.8e10 on: its K is split S ways (or not), against the 128 x 64 tiles of the
+// register-streamed GEMM (group size 128) or the MFMA GEMM, which take p passes over
+// the CUs, K split s ways. A pass of the big tiles does four times the work of one of
+// theirs in about 2.7 times the time and adds the partial tiles, so that the ratio S p
+// / s decides (us, register-streamed / big-tile, 228 shapes measured):
+//   >= 5  768 x 3072 x 14336 (6) 112.5 / 84.6, 384 x 4096 x 18944 (5) 77.0 / 69.1; of 54
+//         shapes the worst is 448 x 3072 x 14336 (5) 53.9 / 55.4;
+//   4     two passes: 1536 x 2048 x 8192 72.1 / 68.1 but 512 x 8192 x 5632 56.7 / 59.9; one:
+//         512 x 4096 x 14336 66.5 / 70.6, except for many rows (2048 x 2048 x 5632 63.9 /
+//         54.1: their activations are read once per 256 columns of y, not per 128);
+//   3     three passes of many rows: 5401 x 844 x 8192 .85 of the time, 1280 x 4096 x 4096
+//         64.4 / 60.6, but 768 x 5632 x 8192 106 / 116; one: 320 x 5632 x 14336 62.2 / 77.2;
+//   2     320 x 11008 x 5632 54.1 / 80.8.
+// The MFMA GEMM (gs 256) is the slower of the two: 768 x 5632 x 8192 (3, three passes)
+// 113 / 103, 512 x 4096 x 14336 (4) 65.3 / 63.9, but 320 x 11008 x 5632 (2) 56.8 / 73.6,
+// 320 x 5632 x 14336 (3, one pass) 64.7 / 74.0.
+bool bgemm_few_tiles(int64_t M, int64_t N, int64_t K, int64_t gs, const pmi::BgemmConfig& b) {
+  if (M * N * K < 18000000000ll) return false;
+  const pmi::Gemm64Config g = pmi::gemm64_config(M, N, K);
+  const int64_t cus = pmi::device_cu_count(), p = (g.grid + cus - 1) / cus, s = g.splits, Sp = b.splits * p;
+  if (!pmi::gemm64_supported(M, K, gs)) return Sp >= 4 * s || p >= 3;
+  return Sp >= 5 * s || (Sp >= 4 * s && (M >= 2048 || (p > 1 && K >= 7168))) ||
+         (p >= 3 && (M >= 2048 || (M >= 1024 && K <= 4096)));
+}
+
 }  // namespace
 
 extern "C" {
@@ -216,14 +242,10 @@ int pmi_matmul_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t group_size
   }
   // Many activation rows (prefill): the big-tile GEMM, 256 weight rows x 128
   // activation rows per workgroup, where its tiles fill three quarters of the
-  // CUs, or, with K split over fewer tiles, from M N K = 1.8e10 on (us, register-
-  // streamed GEMM against it): 4096 x 14336 at M = 256 / 384 / 640 / 1024 39.4 / 56.7
-  // / 109 / 133 against 43.4 / 54.2 / 80 / 112; 4096 x 4096 at M = 1024 / 1152 43.1 / 59.3
-  // against 45.0 / 56.2; 1024 x 14336 at M = 1024 / 1536 38.6 / 63.4 against 41.3 /
-  // 53.8; 7096 x 5504 at M = 512 / 640 50.7 / 73.4 against 51.5 / 74.6.
+  // CUs, or fewer tiles where the other GEMM needs more passes (bgemm_few_tiles).
   if (has_tiled && M > 64 && group_size % 128 == 0 && pmi::tgemm_supported(M, N, K, group_size)) {
     const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, group_size);
-    if (b.ok && ((int64_t)b.n_bands * b.grid_m * 4 >= 3 * cus || M * N * K >= 18000000000ll)) return 6;
+    if (b.ok && ((int64_t)b.n_bands * b.grid_m * 4 >= 3 * cus || bgemm_few_tiles(M, N, K, group_size, b))) return 6;
   }
   // Past 64 rows on narrow layers, while the tiled GEMM's 64-row blocks still
   // take one pass over the CUs: against the register-streamed GEMM, whose K

@@ -104,7 +104,9 @@ PMI_DEV u32x4 descriptor(const void* p, uint32_t bytes) {
 }
 
 // 16 (or 4) bytes per lane from a buffer to LDS address base + 16 (4) * lane.
-// base is uniform. No register is written; the caller waits with wait_vmcnt<0>.
+// base is uniform. No register but m0 is written, which is reserved (a clobber list
+// may not name it): the compiler sets it right ahead of each of its own uses, and
+// has none in this kernel. The caller waits with wait_vmcnt<0>.
 PMI_DEV void dma16(u32x4 r, uint32_t base, int voff, int soff) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(base),

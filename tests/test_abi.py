@@ -289,8 +289,15 @@ def test_pmi_error_maps_to_runtime_error():
     (225, 2060, 2048, 256, True, 3, -1, 6), (130, 516, 1152, 64, True, 2, -1, 6),
     # ... which need room: for the row sums or group-major copies, and for the split
     (64, 4096, 4096, 128, True, 0, 0, 1), (64, 4096, 4096, 64, False, 0, 0, 1),
-    (301, 4096, 14336, 64, False, 1, 0, 5), (643, 2060, 14336, 128, False, 1, 0, 4),
+    (301, 4096, 14336, 64, False, 1, 0, 5), (639, 2060, 14336, 128, False, 1, 0, 4),
     (1024, 1024, 18944, 128, False, 0, 8 << 20, 4),
+    # few tiles (S p / s against the register-streamed GEMM, and the MFMA GEMM at gs 256)
+    (639, 2060, 14336, 128, False, 1, -1, 6), (643, 2060, 14336, 128, False, 1, -1, 4),
+    (320, 11008, 5632, 128, False, 1, -1, 4), (320, 5632, 14336, 128, False, 1, -1, 4),
+    (512, 4096, 14336, 128, False, 1, -1, 4), (512, 8192, 5632, 128, False, 1, -1, 4),
+    (1536, 2048, 8192, 128, False, 1, -1, 6), (2048, 2048, 5632, 128, False, 1, -1, 6),
+    (1280, 4096, 4096, 128, False, 1, -1, 6), (768, 5632, 8192, 128, False, 1, -1, 4),
+    (768, 5632, 8192, 256, False, 1, -1, 6), (320, 5632, 14336, 256, False, 1, -1, 2),
     # unsplit in the GEMV's place where its launches cost more
     (17, 512, 14336, 128, True, 4, 1 << 20, 1), (256, 512, 14336, 128, True, 4, 1 << 20, 6),
     (32, 4096, 4096, 64, False, 0, 2 << 20, 1), (64, 4096, 4096, 64, False, 0, 2 << 20, 6),
