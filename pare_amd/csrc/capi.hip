@@ -540,9 +540,12 @@ bool bgemm_over_gemv(int64_t M, int64_t N, int64_t K) {
 // 24.6 / 35.5; 1024 x 4096 at M = 512 / 768 21.4 / 33.0 against 24.3 / 24.5; 4096 x
 // 14336 at M = 65 / 512 50 / 227 against 30 / 81; 14336 x 4096 at M = 256 54.8
 // against 58.5 (a third block of 112 rows nearly empty), at M = 384 82 against 61.
+// Long rows and too many tiles to split K: from three passes of 128 x 64 tiles on
+// (158 x 17444 x 16384, two passes, 173 against 212; 116 x 23144 x 9728 83 against 96; gs
+// 32, 291 x 8488 x 13312 166 against 196; three: 286 x 13980 x 12288 202 against 185).
 bool bgemm_over_tgemm(int64_t M, int64_t N, int64_t K, const pmi::BgemmConfig& b) {
   if (M <= 64 || M * N * K < 3000000000ll) return false;
-  if (K > 8192) return true;
+  if (K > 8192) return b.splits > 1 || M > 384 || (N + 127) / 128 * ((M + 63) / 64) > 2 * pmi::device_cu_count();
   if (M < 192) return false;
   return (int64_t)b.n_bands * b.grid_m * 2 <= pmi::device_cu_count() || M > 384 ||
          (int64_t)b.grid_m * 16 * b.mt * 5 <= 6 * M;

@@ -298,6 +298,9 @@ def test_pmi_error_maps_to_runtime_error():
     (1536, 2048, 8192, 128, False, 1, -1, 6), (2048, 2048, 5632, 128, False, 1, -1, 6),
     (1280, 4096, 4096, 128, False, 1, -1, 6), (768, 5632, 8192, 128, False, 1, -1, 4),
     (768, 5632, 8192, 256, False, 1, -1, 6), (320, 5632, 14336, 256, False, 1, -1, 2),
+    # long rows, tiles for more than half of the CUs: two passes of the tiled GEMM, three
+    (158, 17444, 16384, 64, False, 1, -1, 5), (291, 8488, 13312, 32, False, 1, -1, 5),
+    (286, 13980, 12288, 32, False, 1, -1, 6), (150, 12532, 8704, 64, False, 1, -1, 6),
     # unsplit in the GEMV's place where its launches cost more
     (17, 512, 14336, 128, True, 4, 1 << 20, 1), (256, 512, 14336, 128, True, 4, 1 << 20, 6),
     (32, 4096, 4096, 64, False, 0, 2 << 20, 1), (64, 4096, 4096, 64, False, 0, 2 << 20, 6),
