@@ -555,12 +555,22 @@ bool bgemm_over_tgemm(int64_t M, int64_t N, int64_t K, const pmi::BgemmConfig& b
 // (us). With the group-major copies: 14336 x 4096 at M = 384 / 512 60.5 / 90 against
 // 64.5 / 66.9, so from tiles for three quarters of the CUs. Without them (which
 // slows that kernel, and costs the big-tile GEMM a 3-5 us launch that makes
-// them): 4096 x 4096 at M = 512 / 768 28.7 / 53 against 33 / 45, 14336 x 4096 at
-// M = 256 / 384 52 / 78 against 47 / 64.5, 4096 x 14336 at M = 256 / 384 47 / 74.5
-// against 44 / 58.8.
+// them): 4096 x 4096 at M = 512 28.7 against 33, 14336 x 4096 at M = 384 78 against
+// 64.5, 4096 x 14336 at M = 384 74.5 against 58.8, from M N K = 2^34 (the line could
+// lie lower: 4096 x 4096 at M = 768 53 against 45, 14336 x 4096 and 4096 x 14336 at M =
+// 256 52 and 47 against 47 and 44). Unsplit, up to 1023 rows, empty rows of the last
+// row block cost more than the passes saved: 152 x 24980 x 18432 (three passes of that
+// GEMM, 152 of 256 rows) 229 against 269, 266 x 19140 x 6656 91 against 103, 404 x 18056 x
+// 5632 (four, 404 of 512) 116 against 125, 313 x 14404 x 5632 (three, 313 of 384) 87
+// against 90; 430 x 15172 x 13312 (four, 430 of 512) 228 against 205, 316 x 26536 x 5120
+// (five) 118 against 114, 1549 x 3264 x 7680 (three) 121 against 115.
 bool bgemm_over_gemm64(int64_t M, int64_t N, int64_t K, bool has_gm, const pmi::BgemmConfig& b) {
   if (M <= 64) return false;
-  if (has_gm) return (int64_t)b.n_bands * b.grid_m * 4 >= 3 * pmi::device_cu_count();
+  const int64_t cus = pmi::device_cu_count(), p = (pmi::gemm64_config(M, N, K).grid + cus - 1) / cus;
+  const int64_t rows = (int64_t)b.grid_m * 16 * b.mt;
+  if (b.splits == 1 && M < 1024 && ((p < 5 && 10 * M < 8 * rows) || (p < 4 && K > 4096 && 10 * M < 9 * rows)))
+    return false;
+  if (has_gm) return (int64_t)b.n_bands * b.grid_m * 4 >= 3 * cus;
   return M * N * K > (1ll << 34);
 }
 

@@ -301,6 +301,10 @@ def test_pmi_error_maps_to_runtime_error():
     # long rows, tiles for more than half of the CUs: two passes of the tiled GEMM, three
     (158, 17444, 16384, 64, False, 1, -1, 5), (291, 8488, 13312, 32, False, 1, -1, 5),
     (286, 13980, 12288, 32, False, 1, -1, 6), (150, 12532, 8704, 64, False, 1, -1, 6),
+    # no tiled copy, unsplit: passes of the register-streamed GEMM and empty rows of blocks
+    (152, 24980, 18432, 128, False, 4, -1, 4), (404, 18056, 5632, 128, False, 0, -1, 4),
+    (430, 15172, 13312, 128, False, 4, -1, 6), (316, 26536, 5120, 128, False, 4, -1, 6),
+    (1549, 3264, 7680, 128, False, 0, -1, 6), (313, 14404, 5632, 128, False, 0, -1, 4),
     # unsplit in the GEMV's place where its launches cost more
     (17, 512, 14336, 128, True, 4, 1 << 20, 1), (256, 512, 14336, 128, True, 4, 1 << 20, 6),
     (32, 4096, 4096, 64, False, 0, 2 << 20, 1), (64, 4096, 4096, 64, False, 0, 2 << 20, 6),
