@@ -531,8 +531,11 @@ size_t tgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size
 // big-tile): 4096 x 4096 gs 64 at M = 16 / 20 / 28 22 / 27.5 / 38 against 19.3; bf16
 // 20 / 26 / 36 against 21; 1024 x 4096 gs 64 bf16 19 / 23 / 32 against 19.3; 14336 x
 // 4096 gs 64 at M = 13 / 24 50 / 85 against 27; 4096 x 14336 bf16 50 / 84 against 30.
-bool bgemm_over_gemv(int64_t M, int64_t N, int64_t K) {
-  return M > 16 || (M >= 12 && N * K >= (1ll << 25));
+// 32-column groups, which it folds four times a unit, on small weights from 21 rows
+// (18 x 660 x 1408 17.8 against 19.7, 18 x 1200 x 896 17.7 against 19.1; 19 x 1688 x 3072 31
+// against 19).
+bool bgemm_over_gemv(int64_t M, int64_t N, int64_t K, int64_t gs) {
+  return M > (gs == 32 && N * K < (1ll << 21) ? 20 : 16) || (M >= 12 && N * K >= (1ll << 25));
 }
 
 // Group sizes 32 and 64 on the tiled copy, past 64 rows (tiled GEMM / big-tile,
@@ -581,7 +584,7 @@ bool use_bgemm(int choice, bool bf16, bool tiled, bool gm, int64_t M, int64_t N,
   if (M < 12 || (!tiled && gs != 32 && gs != 64 && gs != 128)) return false;
   const pmi::BgemmConfig b = pmi::bgemm_config(M, N, K, gs, bf16);
   if (!b.ok) return false;
-  if (bf16 || choice == 1) return bgemm_over_gemv(M, N, K);
+  if (bf16 || choice == 1) return bgemm_over_gemv(M, N, K, gs);
   if (choice == 5) return tiled && gs < 128 && bgemm_over_tgemm(M, N, K, b);
   return (choice == 2 || choice == 4) && gs == 128 && !tiled && bgemm_over_gemm64(M, N, K, gm, b);
 }

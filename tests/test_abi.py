@@ -305,6 +305,9 @@ def test_pmi_error_maps_to_runtime_error():
     (152, 24980, 18432, 128, False, 4, -1, 4), (404, 18056, 5632, 128, False, 0, -1, 4),
     (430, 15172, 13312, 128, False, 4, -1, 6), (316, 26536, 5120, 128, False, 4, -1, 6),
     (1549, 3264, 7680, 128, False, 0, -1, 6), (313, 14404, 5632, 128, False, 0, -1, 4),
+    # 32-column groups on small weights: from 21 rows
+    (18, 660, 1408, 32, True, 4, -1, 1), (18, 1200, 896, 32, False, 0, -1, 1),
+    (21, 660, 1408, 32, True, 4, -1, 6), (19, 1688, 3072, 32, False, 0, -1, 6),
     # unsplit in the GEMV's place where its launches cost more
     (17, 512, 14336, 128, True, 4, 1 << 20, 1), (256, 512, 14336, 128, True, 4, 1 << 20, 6),
     (32, 4096, 4096, 64, False, 0, 2 << 20, 1), (64, 4096, 4096, 64, False, 0, 2 << 20, 6),
