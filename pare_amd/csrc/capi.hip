@@ -554,27 +554,26 @@ bool bgemm_over_tgemm(int64_t M, int64_t N, int64_t K, const pmi::BgemmConfig& b
          (int64_t)b.grid_m * 16 * b.mt * 5 <= 6 * M;
 }
 
-// 128-column groups without the tiled copy, against the register-streamed GEMM
-// (us). With the group-major copies: 14336 x 4096 at M = 384 / 512 60.5 / 90 against
-// 64.5 / 66.9, so from tiles for three quarters of the CUs. Without them (which
-// slows that kernel, and costs the big-tile GEMM a 3-5 us launch that makes
-// them): 4096 x 4096 at M = 512 28.7 against 33, 14336 x 4096 at M = 384 78 against
-// 64.5, 4096 x 14336 at M = 384 74.5 against 58.8, from M N K = 2^34 (the line could
-// lie lower: 4096 x 4096 at M = 768 53 against 45, 14336 x 4096 and 4096 x 14336 at M =
-// 256 52 and 47 against 47 and 44). Unsplit, up to 1023 rows, empty rows of the last
-// row block cost more than the passes saved: 152 x 24980 x 18432 (three passes of that
-// GEMM, 152 of 256 rows) 229 against 269, 266 x 19140 x 6656 91 against 103, 404 x 18056 x
-// 5632 (four, 404 of 512) 116 against 125, 313 x 14404 x 5632 (three, 313 of 384) 87
-// against 90; 430 x 15172 x 13312 (four, 430 of 512) 228 against 205, 316 x 26536 x 5120
-// (five) 118 against 114, 1549 x 3264 x 7680 (three) 121 against 115.
+// 128-column groups without the tiled copy, against the register-streamed GEMM: with
+// the group-major copies from tiles for three quarters of the CUs, without them
+// (which slows that kernel, and costs the big-tile GEMM a 3-5 us launch that makes
+// them) from M N K = 2^34 (the line could lie lower: 4096 x 4096 at M = 768 53 against
+// 45 us), and by the passes over the CUs: p of that GEMM's 128 x 64 tiles, K split s
+// ways, and W of the big tiles, split S ways. From a ratio v = (p / s) / (W / S) on the
+// big tiles win (us, register-streamed / big-tile; of 500 shapes 5 then lose 3-11 %):
+//   split                4    159 x 10488 x 15872 (3) 91 / 103, 278 x 6452 x 9728 (3) 55 / 70
+//   W = 1, no copies     3    384 x 14336 x 4096 (3) 78 / 65, mean of v = 2 .. 1.37 of the time
+//   W = 1, copies        4    152 x 24980 x 18432 (3) 229 / 269, mean of v = 3 .. 1.12
+//   W > 1              2.5    427 x 18440 x 4608 (2) 103 / 111, 996 x 10204 x 4096 (2.5) 104 / 92
+//   W > 2, copies        3    576 x 28024 x 2560 (2.7) 117 / 124
 bool bgemm_over_gemm64(int64_t M, int64_t N, int64_t K, bool has_gm, const pmi::BgemmConfig& b) {
   if (M <= 64) return false;
-  const int64_t cus = pmi::device_cu_count(), p = (pmi::gemm64_config(M, N, K).grid + cus - 1) / cus;
-  const int64_t rows = (int64_t)b.grid_m * 16 * b.mt;
-  if (b.splits == 1 && M < 1024 && ((p < 5 && 10 * M < 8 * rows) || (p < 4 && K > 4096 && 10 * M < 9 * rows)))
-    return false;
-  if (has_gm) return (int64_t)b.n_bands * b.grid_m * 4 >= 3 * cus;
-  return M * N * K > (1ll << 34);
+  const pmi::Gemm64Config g = pmi::gemm64_config(M, N, K);
+  const int64_t cus = pmi::device_cu_count(), tiles = (int64_t)b.n_bands * b.grid_m;
+  if (has_gm ? tiles * 4 < 3 * cus : M * N * K <= (1ll << 34)) return false;
+  const int64_t p = (g.grid + cus - 1) / cus, W = (tiles * b.splits + cus - 1) / cus;
+  const int64_t twice = b.splits > 1 ? 8 : (W == 1 ? (has_gm ? 8 : 6) : (has_gm && W > 2 ? 6 : 5));
+  return 2 * p * b.splits >= twice * W * g.splits;
 }
 
 // Whether a call whose kernel is otherwise `choice` runs on the big-tile GEMM;

@@ -301,10 +301,11 @@ def test_pmi_error_maps_to_runtime_error():
     # long rows, tiles for more than half of the CUs: two passes of the tiled GEMM, three
     (158, 17444, 16384, 64, False, 1, -1, 5), (291, 8488, 13312, 32, False, 1, -1, 5),
     (286, 13980, 12288, 32, False, 1, -1, 6), (150, 12532, 8704, 64, False, 1, -1, 6),
-    # no tiled copy, unsplit: passes of the register-streamed GEMM and empty rows of blocks
+    # no tiled copy: passes of the register-streamed GEMM against those of the big tiles
     (152, 24980, 18432, 128, False, 4, -1, 4), (404, 18056, 5632, 128, False, 0, -1, 4),
     (430, 15172, 13312, 128, False, 4, -1, 6), (316, 26536, 5120, 128, False, 4, -1, 6),
-    (1549, 3264, 7680, 128, False, 0, -1, 6), (313, 14404, 5632, 128, False, 0, -1, 4),
+    (1549, 3264, 7680, 128, False, 0, -1, 6), (159, 10488, 15872, 128, False, 0, -1, 4),
+    (576, 28024, 2560, 128, False, 4, -1, 4), (996, 10204, 4096, 128, False, 4, -1, 6),
     # 32-column groups on small weights: from 21 rows
     (18, 660, 1408, 32, True, 4, -1, 1), (18, 1200, 896, 32, False, 0, -1, 1),
     (21, 660, 1408, 32, True, 4, -1, 6), (19, 1688, 3072, 32, False, 0, -1, 6),
