@@ -439,10 +439,12 @@ class DecoderLayer(nn.Module):
                                             gu._group_size(), gu.out_features)
             return self.down(act.reshape(B, T, -1))
         if M > 64 and gu.use_kernel and gu.g_idx is None and gu.bias is None and \
+                not gu._forward_hooks and not gu._forward_pre_hooks and \
                 kernel_choice(M, gu.out_features, gu.in_features, gu._group_size(), tiled=True) == "bgemm" and \
                 gate_up_silu_rows_supported(M, gu.out_features, gu.in_features, gu._group_size()) and \
                 (self._glu_ready() or not torch.cuda.is_current_stream_capturing()):
-            # a prompt on the big-tile GEMM: the same in its epilogue
+            # a prompt on the big-tile GEMM: the same in its epilogue (a hook on the
+            # linear sees its input and output: the module is then called)
             w_t, sz = self._glu_buffers()
             act = matmul_w4a16_gate_up_silu_rows(n2.reshape(M, -1).contiguous(), w_t, sz,
                                                  gu._group_size(), gu.out_features)

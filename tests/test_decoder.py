@@ -684,3 +684,35 @@ def test_gate_up_silu_rows_equals_matmul_then_silu(M, F, K):
                                          P.sz_group_major(s[idx].contiguous(), z[idx].contiguous()), 128, N)
     assert torch.equal(got.view(torch.int16), silu_mul(y).view(torch.int16))
     assert not gate_up_silu_rows_supported(64, N, K, 128) and not gate_up_silu_rows_supported(M, N, K, 64)
+
+
+def test_hooks_on_the_gate_up_linear_see_a_prompt():
+    """A forward hook (calibration, tracing) on the fused gate/up linear fires for
+    a prompt that the big-tile GEMM's gated epilogue would take, with the same MLP
+    output."""
+    from pare_amd.decoder import DecoderLayer
+    from pare_amd.kernels import gate_up_silu_rows_supported
+
+    cfg = DecoderConfig(hidden=2048, heads=16, kv_heads=8, ffn=8192)
+    layer = DecoderLayer(cfg, torch.Generator(device=DEV).manual_seed(1), DEV)
+    B, T = 1, 512
+    gu = layer.gate_up.fused
+    assert gate_up_silu_rows_supported(B * T, gu.out_features, gu.in_features, 128)
+    cos, sin = rope_tables(cfg.head_dim, cfg.rope_theta, T, DEV)
+    cache = torch.zeros(2, B, cfg.kv_heads, T, cfg.head_dim, dtype=torch.float16, device=DEV)
+    x = torch.randn(B, T, cfg.hidden, generator=torch.Generator(device=DEV).manual_seed(2), device=DEV).half()
+    pos = torch.arange(T, device=DEV)
+
+    def run():
+        with torch.no_grad():
+            return layer.forward_fused(x, None, cos, sin, cache[0], cache[1], pos, True)
+
+    plain = run()
+    seen = []
+    pre = gu.register_forward_pre_hook(lambda m, a: seen.append(a[0].shape))
+    post = gu.register_forward_hook(lambda m, a, y: seen.append(y.shape))
+    hooked = run()
+    pre.remove(), post.remove()
+    assert seen == [(B, T, 2048), (B, T, 16384)]
+    for a, b in zip(plain, hooked):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
