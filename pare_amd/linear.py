@@ -188,7 +188,7 @@ class QuantizedLinear(nn.Module):
         dict: as attributes they go through ``nn.Module.__getattr__``."""
         d = self.__dict__
         cache = d.get("_kernel_cache")
-        if cache is None:
+        if cache is None or len(cache) != 5:   # (a module saved before the cache held five)
             return None
         b = self._buffers
         packed, scale, zero = b["packed_weight"], b["scale"], b["zero"]

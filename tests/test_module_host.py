@@ -128,3 +128,13 @@ def test_kernel_available_needs_the_host_extension(monkeypatch):
 
     monkeypatch.setattr(_lib, "host", missing)
     assert not KN.kernel_available()
+
+
+def test_cache_of_a_module_saved_by_an_earlier_version():
+    """A pickled module carries its kernel copies. One saved when the cache had no
+    tiled_supported entry is left to the general path, which reads four entries."""
+    layer = _ql(64, 256)
+    layer._packed_weight_kernel, layer._packed_weight_tiled, layer._perm16 = layer.packed_weight, None, None
+    layer._kernel_cache = (layer._stamp(), torch.zeros(64, 2, dtype=torch.uint8), None, None)
+    assert layer._forward_host(torch.zeros(1, 256)) is None
+    assert layer._kernel_buffers()[0] is layer.packed_weight
