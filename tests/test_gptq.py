@@ -501,3 +501,50 @@ def test_block_kernel_bit_exact_edges(N, K, b0, count):
     assert np.array_equal(codes[b0:b0 + count].cpu().numpy(), Q)
     assert not codes[:b0].any() and not codes[b0 + count:].any()
     assert np.array_equal(err.cpu().numpy().view(np.uint32), E.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["w inf", "w -inf", "w nan", "w huge", "w tiny", "s 0", "s denormal", "s inf", "s huge",
+                                  "C diag 0", "C diag denormal", "C diag 1e38", "C large updates", "z huge"])
+def test_block_kernel_divides_where_reciprocals_do_not_reach(what):
+    """Infinities, NaN, zero, denormal and overflowing operands: codes and errors
+    are those of the divisions (a NaN code is 0, as the kernel's clamp makes it)."""
+    N, K, gs = 48, 144, 16
+    rng = np.random.default_rng(5)
+    W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    C = np.triu(rng.standard_normal((K, K)) * 0.05).astype(np.float32)
+    C[np.arange(K), np.arange(K)] = rng.uniform(0.3, 3.0, K).astype(np.float32)
+    colg = np.arange(K, dtype=np.int32) // gs
+    scale = rng.uniform(1e-3, 6e-3, (N, K // gs)).astype(np.float32)
+    zero = rng.integers(0, 16, (N, K // gs)).astype(np.float32)
+    special = {"inf": np.inf, "-inf": -np.inf, "nan": np.nan, "huge": 1e38, "tiny": 1e-39, "0": 0.0,
+               "denormal": 1e-40, "1e38": 1e38, "updates": 1e38}[what.split()[-1]]
+    if what[0] == "w":
+        W[[3, 20], 40] = special
+    elif what[0] == "s":
+        scale[[3, 20], 2] = special
+    elif what[0] == "z":
+        zero[[3, 20], 2] = special
+    elif "diag" in what:
+        C[40, 40] = special
+    else:
+        C[40, 44:] = special
+    E = np.zeros((128, N), np.float32)
+    Q = np.zeros((128, N), np.uint8)
+    Wb = W[:, :128].copy()
+    with np.errstate(all="ignore"):
+        for k in range(128):
+            s, z = scale[:, colg[k]], zero[:, colg[k]]
+            q = np.fmin(np.fmax(np.rint(Wb[:, k] / s + z), np.float32(0)), np.float32(15))
+            e = (Wb[:, k] - (q - z) * s) / C[k, k]
+            Q[k], E[k] = q, e
+            Wb[:, k + 1:] -= e[:, None] * C[k, k + 1:128][None, :]
+    d = [torch.from_numpy(a).to("cuda") for a in (W, C, colg, scale, zero)]
+    codes = torch.zeros(K, N, dtype=torch.uint8, device="cuda")
+    err = torch.zeros(128, N, device="cuda")
+    rc = _lib.lib().pmi_gptq_block(*(v.data_ptr() for v in d), codes.data_ptr(), err.data_ptr(), N, K,
+                                   K // gs, 0, 128, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(codes[:128].cpu().numpy(), Q)
+    assert np.array_equal(err.cpu().numpy(), E, equal_nan=True)
