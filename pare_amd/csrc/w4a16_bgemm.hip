@@ -52,6 +52,13 @@
 // 0x64 exponent byte, one packed subtract); the products x (q - z) are exact in
 // fp32; y += s * sum x (q - z) per group in fp32, the reference's w = (q - z) * s
 // with fp32 accumulation (pare/kernels/matmul_int4.py:145-176).
+// bf16: products x (128 + q) are exact as well, but a group's sum and its start are up
+// to 143 |x| a term and cancel, as they do in the GEMV and the tiled GEMM's bf16
+// variant: each of their roundings is 2^-24 of that. Below the rounding of y to bf16
+// (1.7e-3) unless a column is some 10^4 times the others: against 64 bits, 64 x 512 x
+// 4096, N(0, 1) activations, or those with a mean of 100, 1.65e-3 and 1.72e-3, the
+// rounding itself; with two columns of 1e3 / 1e4 / 1e5 whose codes equal their zero
+// points 1.66e-3 / 1.71e-3 / 4.1e-3 (the GEMV 1.66e-3 / 1.76e-3 / 6.0e-3).
 #include <atomic>
 
 #include "pmi_common.h"

@@ -107,6 +107,35 @@ def test_bgemm_routes_against_fp64_and_the_gemv(M, N, K, gs, bf16, copies, act_o
     assert (diff <= 2 * bound).all(), f"against the GEMV: {np.max(diff / bound):.2f} of the bound"
 
 
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("what", ["mean", "outlier"])
+def test_bgemm_bf16_under_cancellation(gs, what):
+    """Activations with a large common offset, and outlier columns whose codes equal
+    their zero points: products with 128 + q that cancel against the row sums.
+    They are about 2^-24 143 max|x| s of error per rounding, a dozen roundings a
+    group: against sums of sqrt(K) 4.6 s (offset 100: 100 times that) below 2e-4
+    of y, where its rounding to bf16 is 1.7e-3 of it, so 2 % beside that."""
+    M, N, K = 96, 516, 4096
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q = torch.randint(0, 16, (N, K), generator=g, device=DEV, dtype=torch.uint8)
+    z = torch.randint(0, 16, (N, K // gs), generator=g, device=DEV, dtype=torch.uint8)
+    s = torch.rand(N, K // gs, generator=g, device=DEV) * 0.004 + 0.001
+    x = torch.randn(M, K, generator=g, device=DEV)
+    if what == "mean":
+        x += 100.0
+    else:
+        for c in (5, gs + 3):
+            q[:, c], x[:, c] = z[:, c // gs], 1000.0
+    x = x.bfloat16()
+    wk = P.repack_int4_for_kernel(q[:, 0::2] | (q[:, 1::2] << 4), gs)
+    w = ((q.double().reshape(N, -1, gs) - z.double()[..., None]) * s.double()[..., None]).reshape(N, K)
+    ref = x.double() @ w.t()
+    assert kernel_route(M, N, K, gs, torch.bfloat16) == "bgemm"
+    y = P.matmul_w4a16_bf16(x, wk, s, z, gs).double()
+    rounding = (ref.bfloat16().double() - ref).norm()
+    assert (y - ref).norm() <= 1.02 * rounding
+
+
 def test_bgemm_route_needs_no_workspace_and_no_alignment_of_y():
     """With no workspace, or a y that is not 8-byte aligned, bf16 calls of many
     rows run on the GEMV as before, through the C ABI."""
