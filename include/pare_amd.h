@@ -160,8 +160,9 @@ PMI_API int pmi_tile_w4a16(const uint8_t* w_kernel, uint8_t* w_tiled, int64_t N,
  * reference casts bf16 activations to fp16, pare/layers/linear.py:154-156;
  * y rounded to bf16; with w_tiled and no perm, the rows an fp16 call would
  * run on the tiled GEMM's 16-row blocks take its bf16 variant (one K range,
- * group_size % 128 == 0), the rest run on the GEMV, four activation rows per
- * launch, and with perm it needs the workspace for the gather of X[:, perm]);
+ * group_size % 128 == 0), many rows the big-tile GEMM (pmi_matmul_route), the
+ * rest the GEMV, four activation rows per launch; with perm both need the
+ * workspace for the gather of X[:, perm]);
  * zeros: PMI_F32 or PMI_U8 [N,G]; perm (nullable, int32 [K]): act_order
  * gather, X is read as X[:, perm[j]] for weight column j (w must then be
  * repacked with the same perm); y: fp16 [M,N].
@@ -182,16 +183,17 @@ PMI_API int pmi_tile_w4a16(const uint8_t* w_kernel, uint8_t* w_tiled, int64_t N,
  * the kernel it would pick without w_tiled (an error if the tiled GEMM is
  * forced); y needs only 2-byte alignment otherwise.
  * workspace (nullable when workspace_bytes == 0): device scratch of
- * pmi_matmul_workspace_bytes() bytes, 256-byte aligned, zero-filled before
- * its first use; every call leaves it zero-filled again (it holds split-K
- * counters, partial tiles and the act_order gather of X). A smaller or null
+ * pmi_matmul_workspace_bytes() bytes, 256-byte aligned, its first 64 KiB (the
+ * split-K counters) zero-filled before its first use; every call leaves them
+ * zero again (partial tiles and the act_order gather of X follow). A smaller or null
  * workspace is accepted: the GEMM then runs without split-K, and act_order
  * shapes fall back to the GEMV. With pmi_matmul_best_workspace_bytes() bytes,
  * row counts past 11 that would stream the weights once per four (GEMV) or 64
  * rows (bf16, group sizes 32 and 64, K % 256 != 0, callers without w_tiled) run
  * on the big-tile GEMM where that wins (N % 4 == 0, K % 128 == 0, y 8-byte
- * aligned). Calls that may run concurrently (other
- * streams) must not share a workspace.
+ * aligned; pmi_matmul_route). Calls that may run concurrently (other streams,
+ * replays of captured graphs) or whose launches may interleave (other threads on
+ * one stream) must not share a workspace.
  * Requires K % group_size == 0, group_size % 32 == 0, K % 32 == 0.
  * Replaces: matmul_w4a16(x, packed_weight, scales, zeros, group_size)
  *           pare/kernels/matmul_int4.py:183-243 (kernel :66-176) */

@@ -234,9 +234,11 @@ def matmul_w4a16_bf16(
     which ``matmul_w4a16`` keeps. Here the bf16 values are used as they are
     (fp32 accumulation, y rounded to bf16): with ``w_tiled`` and ``sz_gm`` and
     no ``perm``, the row counts an fp16 call runs on the tiled GEMM's 16-row
-    blocks take its bf16 variant; more than 16 rows (11 on large layers) run on
-    the big-tile GEMM (N % 4 == 0, K % 128 == 0), the rest on the GEMV, four
-    activation rows per launch. Other arguments as for ``matmul_w4a16``."""
+    blocks take its bf16 variant; more than 16 rows (11 on large layers, 20 on
+    small ones of 32-column groups) run on the big-tile GEMM (N % 4 == 0, K % 128
+    == 0; groups of 256 and more with ``w_tiled``), with or without ``perm``, the
+    rest on the GEMV, four activation rows per launch. Other arguments as for
+    ``matmul_w4a16``."""
     if not x.is_cuda:
         raise RuntimeError("matmul_w4a16_bf16 requires HIP (cuda) tensors.")
     assert x.is_contiguous(), "x must be contiguous"
