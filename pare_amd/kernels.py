@@ -206,7 +206,8 @@ def matmul_w4a16(
         raise RuntimeError("matmul_w4a16 requires HIP (cuda) tensors.")
     assert x.is_contiguous(), "x must be contiguous"
     assert x.dtype == torch.float16, f"x must be float16, got {x.dtype}"
-    if out is None and x.dim() == 2 and (sz_gm is None or len(sz_gm) == 2):
+    if out is None and zeros.dtype is torch.uint8 and scales.dtype is torch.float32 and x.dim() == 2 and \
+            (sz_gm is None or len(sz_gm) == 2):
         y = host_matmul(x, packed_weight, scales, zeros, group_size, perm, perm16, sz_gm, w_tiled,
                         bf16=False)
         if y is not None:
@@ -243,7 +244,8 @@ def matmul_w4a16_bf16(
         raise RuntimeError("matmul_w4a16_bf16 requires HIP (cuda) tensors.")
     assert x.is_contiguous(), "x must be contiguous"
     assert x.dtype == torch.bfloat16, f"x must be bfloat16, got {x.dtype}"
-    if out is None and x.dim() == 2 and (sz_gm is None or len(sz_gm) == 2):
+    if out is None and zeros.dtype is torch.uint8 and scales.dtype is torch.float32 and x.dim() == 2 and \
+            (sz_gm is None or len(sz_gm) == 2):
         y = host_matmul(x, packed_weight, scales, zeros, group_size, perm, perm16, sz_gm, w_tiled,
                         bf16=True)
         if y is not None:
