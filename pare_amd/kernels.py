@@ -120,8 +120,8 @@ class _Workspaces(threading.local):
 _workspaces = _Workspaces()
 
 
-def _new_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
-    ws = torch.empty(1 << max(nbytes - 1, (1 << 20) - 1).bit_length(), dtype=torch.uint8, device=dev)
+def _new_workspace(dev: torch.device, nbytes: int, least: int) -> torch.Tensor:
+    ws = torch.empty(1 << (max(nbytes, least) - 1).bit_length(), dtype=torch.uint8, device=dev)
     ws[:_COUNTER_BYTES].zero_()
     return ws
 
@@ -147,13 +147,15 @@ def _workspace(dev: torch.device, stream: int, nbytes: int) -> torch.Tensor | No
         capture = _capture_id(stream)
         last, ws = _workspaces.captured.get(key, (None, None))
         if last != capture or ws.numel() < nbytes:
-            ws = _new_workspace(dev, nbytes)
+            # every growth is another fill of the counters in each replay (2-3 us): 8 MiB
+            # hold a decoder step's calls
+            ws = _new_workspace(dev, nbytes, 8 << 20)
             _workspaces.captured[key] = (capture, ws)
         return ws
     _workspaces.captured.pop(key, None)
     ws = _workspaces.eager.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = _workspaces.eager[key] = _new_workspace(dev, nbytes)
+        ws = _workspaces.eager[key] = _new_workspace(dev, nbytes, 1 << 20)
     return ws
 
 

@@ -68,7 +68,8 @@ def test_workspaces_of_captures_and_eager_calls_are_apart(monkeypatch):
     first = KN._workspace(dev, stream, 1 << 20)
     assert first is not eager and KN._workspace(dev, stream, 1 << 19) is first
     assert first[:64 * 1024].eq(0).all()
-    larger = KN._workspace(dev, stream, (1 << 20) + 1)
+    assert KN._workspace(dev, stream, 8 << 20) is first      # one fill of the counters for small calls
+    larger = KN._workspace(dev, stream, (8 << 20) + 1)
     assert larger is not first and KN._workspace(dev, stream, 1 << 20) is larger
     capture = 12
     second = KN._workspace(dev, stream, 1 << 20)
